@@ -12,7 +12,8 @@
 //     a wave reads bytes [16 L, 16 L + 16) = W[16 g + n][64 c + 16 j .. + 16] with one 16-byte load, so a wave's
 //     load is one contiguous KiB. Within a chunk the contraction index is permuted identically for both operands
 //     (MFMA h = 0, 1 of the chunk takes bytes 8h..8h+7 of every lane), which leaves the dot product unchanged.
-//   * GEMM inputs: bf16 planes [kTerms][16][K]; lane (m + 16 j) reads x[m][64 c + 16 j .. + 16] of every plane.
+//   * GEMM inputs: bf16 planes [kTerms][16][K], row-major at the C interface; the planes that stay inside the batched
+//     step are kept in the order in which the matrix cores take them (plane_index).
 //   * RMSNorm: the kernel that updates the residual h also writes the planes of bf16(h ⊙ w_next) and, per
 //     16-column tile, the partial sums of squares of h; the consuming GEMM adds the partials of its row in a fixed
 //     order and applies rsqrt(Σh²/K + eps) after the dot product (qwen3/kernels.py:180-186, 224).
@@ -35,8 +36,8 @@ constexpr int kM = 16;         // rows of every activation buffer (streams)
 #endif
 constexpr int kTerms = SK_BATCH_TERMS;
 constexpr int kThreads = 256;
+constexpr int kMaxSlices = 4;  // K slices of one GEMM (plan)
 constexpr int kOutF32 = 0, kOutSwiglu = 1, kOutAcc = 2;
-constexpr int kMaxSlices = 16;  // K slices of one GEMM (the plan keeps S = K / (64 CW) at or below this)
 
 // ---- conversions ----------------------------------------------------------------------------------------------
 // two floats whose low 16 bits are zero (small integers) -> packed bf16 pair, lo in the low half
@@ -70,6 +71,22 @@ __device__ __forceinline__ void store_terms(bf16_t* __restrict__ planes, size_t 
   }
 }
 
+// Orders this wave's LDS stores before its later loads of the same words by other lanes (LDS operations of one wave
+// complete in order, so no wait or barrier is needed).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// rotation (in fours) of staging segment s = 2 (j & 1) + h, s = 0..3
+__device__ __forceinline__ int sq_rot(int s) { return 2 * ((s >> 1) & 1) + (s & 1); }
+
+// Index of x[m][k] in a plane of K columns: row-major at the C interface; inside the batched step (TILED) in the order in
+// which the matrix cores take it, 1 KiB per (64-wide chunk, half h): lane m + 16 j holds x[m][64 c + 16 j + 8 h .. + 8].
+template <bool TILED>
+__device__ __forceinline__ size_t plane_index(int m, int k, int K) {
+  return TILED ? (size_t)((k >> 6) * 2 + ((k >> 3) & 1)) * 512 + (((k >> 4) & 3) * 16 + m) * 8 + (k & 7) : (size_t)m * K + k;
+}
+
 struct GemmArgs {
   const bf16_t* x;      // input planes [kTerms][16][K]
   const float* ssp;     // [np][16] partial sums of squares behind x (NULL: no RMSNorm scale)
@@ -83,161 +100,193 @@ struct GemmArgs {
   bf16_t* xn;           // ACC: planes [kTerms][16][N] of bf16(h ⊙ nw)
   const float* nw;      // ACC: next RMSNorm weight [N]
   float* ssp_out;       // ACC: [N/16][16] partial sums of squares of the updated residual
-  int S;                // K slices (workgroups per row block)
-  float* part;          // S > 1: [S][N / 16][256] partial sums
-  unsigned* counters;   // S > 1: [row blocks] arrivals, zero between launches
+  int S = 1;            // K slices (workgroups per row block)
+  float* part = nullptr;          // S > 1: [S][N / 16][256] partial sums
+  unsigned* counters = nullptr;   // S > 1: [row blocks] arrivals, zero between launches
 };
 
-// Workgroup (nb, slice) computes output row groups 4 R nb .. 4 R nb + 4 R - 1 (16 rows each; wave w owns R of them)
-// for all 16 streams over K slice `slice` (CW chunks of 64). The slice's activation planes are read from memory once
-// per workgroup into LDS and shared by the four waves, which split the rows: the planes' traffic is then one read
-// per 64 R output rows instead of one per 16 R (when the waves split K instead, each workgroup read its whole slice
-// for 16 R rows, and the planes of a step were read 2-3 times more often than the weights). Every load goes out at
-// the top: the activation slice first (it is needed first), then the wave's weights (its HBM traffic). With S > 1
-// slices the workgroups of a row block publish their sums (device-coherent stores) and the last to arrive adds them in
-// slice order and runs the epilogue, so the result does not depend on arrival order.
-template <int OUT, int R, int CW>
-__global__ __launch_bounds__(kThreads) void k_bgemm(GemmArgs p) {
-  constexpr int kSeg = kTerms * kM * CW * 8;            // 16-byte activation segments of the slice
-  constexpr int kAct = (kSeg + kThreads - 1) / kThreads;  // per thread
-  __shared__ uint4 xs[kTerms][CW][2][64];  // [term][chunk][half][lane m + 16 j]: bf16 x[m][64 c + 16 j + 8 h ..+8]
-  __shared__ float ssq[16][kM];
-  __shared__ float inv_s[kM];
+// Workgroup (nb, slice) computes RG row groups (16 output rows each) for all 16 streams over K slice `slice`, which its
+// kWaves waves split once more (wave w takes KW chunks of 64), each for all RG groups; the waves' sums meet once in LDS
+// and are added in wave order. What bounds it is latency, not a rate: the launch (2.2-2.6 us measured with every load
+// and MFMA taken out), then one memory round trip, since every load a wave will make goes out at the top: the weights
+// (from HBM) first, then the activation planes (from L2). Weights first measured 5.7 against 6.2 us (qkv 4096 x 2048),
+// 4.8 against 5.5 (o 2048 x 2048) and 5.8 against 7.1 (down 1024 x 3072) for chunk by chunk.
+//   * Up to K = 2048 a workgroup takes all of K, so nothing is exchanged between workgroups. Splitting K over workgroups
+//     for every shape (partial sums stored, acknowledged, counted and reloaded before the epilogue) took 9.2 / 7.5 /
+//     16.6 us (qkv / o / gate-up 12288 x 2048) against 5.8 / 4.9 / 9.0 now.
+//   * Beyond, reading all of the planes (96 K bytes) takes a CU longer than the exchange: K is cut into slices of 1536 or
+//     2048, the workgroups of a row block publish their sums (device-coherent stores) and the last to arrive adds them
+//     in slice order, so the result does not depend on arrival order. Down 2048 x 6144: 10.1 us with 12 slices of 512,
+//     12.3 with the whole of K, 7.2 with 4 of 1536.
+//   * TILED planes (plane_index) are loaded as whole fragments, 1 KiB per instruction. Row-major planes, the C
+//     interface's, are loaded four lanes per row (64 contiguous bytes) and turned into fragments by a trip through 6 KB
+//     of LDS that only this wave uses, so no barrier; the trip costs 1.4 us at K = 2048 (LDS bandwidth).
+template <int OUT, bool TILED, int kWaves, int RG, int KW>
+__global__ __launch_bounds__(64 * kWaves) void k_bgemm(GemmArgs p) {
+  constexpr int kGemmThreads = 64 * kWaves;
+  constexpr int kStrips = RG * 4, kOwn = (kStrips + kWaves - 1) / kWaves;  // 64-element output strips, per wave
+  __shared__ uint4 stage[kWaves][TILED ? kStrips * 16 : kTerms * 128];  // [term][half][lane m + 16 j], one chunk per wave
   __shared__ int last_s;
+  __shared__ float ssq[kGemmThreads / 16][kM];
+  __shared__ float inv_s[kM];
+  static_assert(kWaves * kStrips * 64 * 4 <= (int)sizeof(stage), "the waves' sums alias the staging area");
+  float(*red)[kStrips][64] = (float(*)[kStrips][64])&stage[0][0];  // [wave][strip 4 r + i][lane]
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
   const int C = p.K / 64;                 // 64-wide chunks per row
   const int G = p.N / 16;                 // row groups
-  const int nb = blockIdx.x, slice = blockIdx.y;
-  const int c0 = slice * CW;
-  const int g0 = (nb * 4 + wv) * R;       // this wave's first row group
+  const int g0 = blockIdx.x * RG;
   const size_t plane = (size_t)kM * p.K;
-  // the slice's activation segments: segment a = (t, m, q) holds bf16 x_t[m][64 c0 + 8 q .. + 8]
-  uint4 av[kAct];
+  const int slice = blockIdx.y;
+  const int c0 = (slice * kWaves + wv) * KW;
+  // activation loads: lane 4 m + s takes 16-byte segments s and 4 + s of row m's chunk, per term
+  const bf16_t* xw = TILED ? p.x + (size_t)c0 * 1024 + lane * 8 : p.x + (size_t)(lane >> 2) * p.K + (size_t)c0 * 64 + 8 * (lane & 3);
+  const uint4* wp[RG];
 #pragma unroll
-  for (int i = 0; i < kAct; i++) {
-    const int a = tid + kThreads * i;
-    if (a < kSeg) {
-      const int t = a / (kM * CW * 8), m = (a / (CW * 8)) % kM, q = a % (CW * 8);
-      av[i] = gload4((const uint4*)(p.x + t * plane + (size_t)m * p.K + (size_t)c0 * 64 + 8 * q));
-    }
-  }
-  uint4 wq[CW][R];
+  for (int r = 0; r < RG; r++)  // a row group past the matrix loads the last one (never stored)
+    wp[r] = (const uint4*)p.w + ((size_t)min(g0 + r, G - 1) * C + c0) * 64 + lane;
+  uint4 wq[KW][RG], xq[KW][kTerms][2];
 #pragma unroll
-  for (int c = 0; c < CW; c++)
+  for (int c = 0; c < KW; c++)
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-      const int g = min(g0 + r, G - 1);  // a row group past the matrix loads the last one (never stored)
-      wq[c][r] = ld_stream((const uint4*)p.w + ((size_t)g * C + c0 + c) * 64 + lane);
-    }
+    for (int r = 0; r < RG; r++) wq[c][r] = ld_stream(wp[r] + c * 64);
+  __builtin_amdgcn_sched_barrier(0);  // keep the weights ahead of the planes
+#pragma unroll
+  for (int c = 0; c < KW; c++)
+#pragma unroll
+    for (int t = 0; t < kTerms; t++)
+#pragma unroll
+      for (int i = 0; i < 2; i++) xq[c][t][i] = gload4((const uint4*)(xw + t * plane + (TILED ? 1024 * c + 512 * i : 64 * c + 32 * i)));
   float ssv = 0.f;  // this thread's share of the RMSNorm partial sums
   if (p.ssp)
-    for (int q = tid >> 4; q < p.np; q += 16) ssv += gload(p.ssp + q * kM + (tid & 15));
+    for (int q = tid >> 4; q < p.np; q += kGemmThreads / 16) ssv += gload(p.ssp + q * kM + (tid & 15));
+  // what the epilogue needs of this thread's outputs
+  const int nl = lane & 15;
+  float sc[kOwn], hv[kOwn], nv[kOwn];
 #pragma unroll
-  for (int i = 0; i < kAct; i++) {
-    const int a = tid + kThreads * i;
-    if (a < kSeg) {
-      const int t = a / (kM * CW * 8), m = (a / (CW * 8)) % kM, q = a % (CW * 8);
-      xs[t][q >> 3][q & 1][m + 16 * ((q >> 1) & 3)] = av[i];
+  for (int o = 0; o < kOwn; o++) {
+    const int st = min(wv + o * kWaves, kStrips - 1), g = min(g0 + st / 4, G - 1), n = g * 16 + nl, m = 4 * (lane >> 4) + st % 4;
+    sc[o] = bf2f(gload(p.s + n));
+    if constexpr (OUT == kOutAcc) {
+      hv[o] = gload(p.out + (size_t)m * p.N + n);
+      nv[o] = gload(p.nw + n);
     }
   }
+  f32x4 acc[RG], acc2[RG];  // first term, later terms (kept apart: the small terms accumulate at their own scale)
+#pragma unroll
+  for (int r = 0; r < RG; r++) { acc[r] = f32x4{0.f, 0.f, 0.f, 0.f}; acc2[r] = acc[r]; }
+  uint4* my = &stage[wv][0];
+  // segment q = 2 j + h of row m sits at slot 16 j + (m rotated by 4 (2 (j & 1) + h)) of half h: the 8 lanes of a
+  // store beat and the 8 of a read beat each touch distinct bank groups
+  const int sm = lane >> 2, sq = lane & 3, wslot = (sq & 1) * 64 + 16 * (sq >> 1) + ((sm + 4 * sq_rot(sq)) & 15);
+  const int rj = lane >> 4, rs0 = 16 * rj + ((nl + 8 * (rj & 1)) & 15), rs1 = 64 + 16 * rj + ((nl + 8 * (rj & 1) + 4) & 15);
+#pragma unroll
+  for (int c = 0; c < KW; c++) {
+    bf16x8 xa[kTerms][2];
+    if constexpr (TILED) {
+#pragma unroll
+      for (int t = 0; t < kTerms; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) xa[t][i] = as_bf16x8(xq[c][t][i]);
+    } else {
+#pragma unroll
+      for (int t = 0; t < kTerms; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) my[t * 128 + wslot + 32 * i] = xq[c][t][i];
+      wave_sync();
+#pragma unroll
+      for (int t = 0; t < kTerms; t++) {
+        xa[t][0] = as_bf16x8(my[t * 128 + rs0]);
+        xa[t][1] = as_bf16x8(my[t * 128 + rs1]);
+      }
+      wave_sync();
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int r = 0; r < RG; r++) {
+        const uint4 q = wq[c][r];
+        const bf16x8 b = h ? i8x8_bf16(q.z, q.w) : i8x8_bf16(q.x, q.y);
+        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[0][h], b, acc[r], 0, 0, 0);
+#pragma unroll
+        for (int t = 1; t < kTerms; t++) acc2[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t][h], b, acc2[r], 0, 0, 0);
+      }
+  }
   if (p.ssp) ssq[tid >> 4][tid & 15] = ssv;
-  __syncthreads();
+  __syncthreads();  // every wave is done with its staging area
+  // D[m][n] sits in lane n + 16 (m / 4), element m % 4
+#pragma unroll
+  for (int r = 0; r < RG; r++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) red[wv][4 * r + i][lane] = acc[r][i] + acc2[r][i];
   if (p.ssp && tid < kM) {
     float s = 0.f;
 #pragma unroll
-    for (int q = 0; q < 16; q++) s += ssq[q][tid];
+    for (int q = 0; q < kGemmThreads / 16; q++) s += ssq[q][tid];
     inv_s[tid] = rsqrtf(s / p.K + p.eps);
   }
-  f32x4 acc[R], acc2[R];  // first term, later terms (kept apart: the small terms accumulate at their own scale)
+  __syncthreads();
+  float vs[kOwn];
 #pragma unroll
-  for (int r = 0; r < R; r++) { acc[r] = f32x4{0.f, 0.f, 0.f, 0.f}; acc2[r] = acc[r]; }
+  for (int o = 0; o < kOwn; o++) {
+    const int st = min(wv + o * kWaves, kStrips - 1);
+    vs[o] = red[0][st][lane];
 #pragma unroll
-  for (int c = 0; c < CW; c++) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      bf16x8 xa[kTerms];
-#pragma unroll
-      for (int t = 0; t < kTerms; t++) xa[t] = as_bf16x8(xs[t][c][h][lane]);
-#pragma unroll
-      for (int r = 0; r < R; r++) {
-        const uint4 q = wq[c][r];
-        const bf16x8 b = h ? i8x8_bf16(q.z, q.w) : i8x8_bf16(q.x, q.y);
-        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[0], b, acc[r], 0, 0, 0);
-#pragma unroll
-        for (int t = 1; t < kTerms; t++) acc2[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[t], b, acc2[r], 0, 0, 0);
-      }
-    }
+    for (int w = 1; w < kWaves; w++) vs[o] += red[w][st][lane];
   }
-  // D[m][n] sits in lane n + 16 (m / 4), element m % 4
-  float v[R][4];
-#pragma unroll
-  for (int r = 0; r < R; r++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[r][i] = acc[r][i] + acc2[r][i];
   if (p.S > 1) {
     // partial of (slice, row group g): 256 floats, element i of lane L at 64 i + L
     const uint32_t stride = (uint32_t)G * 256u;
 #pragma unroll
-    for (int r = 0; r < R; r++)
-      if (g0 + r < G)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          buf_stf(p.part, ((uint32_t)slice * stride + (uint32_t)(g0 + r) * 256u + 64u * i + lane) * 4u, v[r][i]);
+    for (int o = 0; o < kOwn; o++) {
+      const int st = wv + o * kWaves;
+      if (st < kStrips && g0 + st / 4 < G)
+        buf_stf(p.part, ((uint32_t)slice * stride + (uint32_t)(g0 * 4 + st) * 64u + lane) * 4u, vs[o]);
+    }
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (tid == 0) {
-      const unsigned prev = __hip_atomic_fetch_add(&p.counters[nb], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const unsigned prev = __hip_atomic_fetch_add(&p.counters[blockIdx.x], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       last_s = prev == (unsigned)(p.S - 1);
     }
     __syncthreads();
     if (!last_s) return;
     // every slice's partial at once (one round trip), then the sum in slice order
-    float pv[kMaxSlices][R][4];
+    float pv[kMaxSlices][kOwn];
 #pragma unroll
     for (int q = 0; q < kMaxSlices; q++)
       if (q < p.S)
 #pragma unroll
-        for (int r = 0; r < R; r++)
+        for (int o = 0; o < kOwn; o++) {
+          const int st = min(wv + o * kWaves, kStrips - 1), g = min(g0 + st / 4, G - 1);
+          pv[q][o] = buf_ldf(p.part, ((uint32_t)q * stride + (uint32_t)(g * 4 + st % 4) * 64u + lane) * 4u);
+        }
 #pragma unroll
-          for (int i = 0; i < 4; i++)
-            pv[q][r][i] = buf_ldf(p.part, ((uint32_t)q * stride + (uint32_t)min(g0 + r, G - 1) * 256u + 64u * i + lane) * 4u);
+    for (int o = 0; o < kOwn; o++) {
+      vs[o] = pv[0][o];
 #pragma unroll
-    for (int r = 0; r < R; r++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        float a = 0.f;
-#pragma unroll
-        for (int q = 0; q < kMaxSlices; q++)
-          if (q < p.S) a += pv[q][r][i];
-        v[r][i] = a;
-      }
-    if (tid == 0) __hip_atomic_store(&p.counters[nb], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  } else {
-    __syncthreads();  // inv_s
+      for (int q = 1; q < kMaxSlices; q++)
+        if (q < p.S) vs[o] += pv[q][o];
+    }
+    if (tid == 0) __hip_atomic_store(&p.counters[blockIdx.x], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  const int nl = lane & 15;
 #pragma unroll
-  for (int r = 0; r < R; r++) {
-    if (g0 + r >= G) break;
-    const int n = (g0 + r) * 16 + nl;
-    const float sc = bf2f(p.s[n]);
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int m = 4 * (lane >> 4) + i;
-      const float y = v[r][i] * sc * (p.ssp ? inv_s[m] : 1.f);
-      if constexpr (OUT == kOutF32) {
-        p.out[(size_t)m * p.N + n] = y;
-      } else if constexpr (OUT == kOutSwiglu) {
-        const float u = dpp<0xB1>(y);  // lane L ^ 1: the up row next to this gate row
-        if (!(nl & 1)) store_terms(p.act, (size_t)kM * (p.N / 2), (size_t)m * (p.N / 2) + n / 2, silu_mul(y, u));
-      } else {
-        float* hp = p.out + (size_t)m * p.N + n;
-        const float hn = *hp + y;
-        *hp = hn;
-        store_terms(p.xn, (size_t)kM * p.N, (size_t)m * p.N + n, hn * p.nw[n]);
-        const float ss = row16_sum(hn * hn);
-        if (nl == 0) p.ssp_out[(g0 + r) * kM + m] = ss;
-      }
+  for (int o = 0; o < kOwn; o++) {
+    const int st = wv + o * kWaves;
+    if (st >= kStrips || g0 + st / 4 >= G) break;
+    const float v = vs[o];
+    const int g = g0 + st / 4, n = g * 16 + nl, m = 4 * (lane >> 4) + st % 4;
+    const float y = v * sc[o] * (p.ssp ? inv_s[m] : 1.f);
+    if constexpr (OUT == kOutF32) {
+      p.out[(size_t)m * p.N + n] = y;
+    } else if constexpr (OUT == kOutSwiglu) {
+      const float u = dpp<0xB1>(y);  // lane L ^ 1: the up row next to this gate row
+      if (!(nl & 1)) store_terms(p.act, (size_t)kM * (p.N / 2), plane_index<TILED>(m, n / 2, p.N / 2), silu_mul(y, u));
+    } else {
+      const float hn = hv[o] + y;
+      p.out[(size_t)m * p.N + n] = hn;
+      store_terms(p.xn, (size_t)kM * p.N, plane_index<TILED>(m, n, p.N), hn * nv[o]);
+      const float ss = row16_sum(hn * hn);
+      if (nl == 0) p.ssp_out[g * kM + m] = ss;
     }
   }
 }
@@ -285,7 +334,11 @@ struct AttnArgs {
   bf16_t* att;          // planes [kTerms][16][nq * 128]
   float* part;          // [batch * nkv][2][kAttnSplitMax][kPart]
   int* err;
+  bool tiled;           // layout of att (plane_index)
 };
+__device__ __forceinline__ size_t att_index(const AttnArgs& a, int b, int k) {
+  return a.tiled ? plane_index<true>(b, k, a.nq * SK_HD) : plane_index<false>(b, k, a.nq * SK_HD);
+}
 
 __device__ __forceinline__ void unpack8(uint4 v, float* o) {
   o[0] = bf2f(v.x & 0xffffu); o[1] = bf2f(v.x >> 16); o[2] = bf2f(v.y & 0xffffu); o[3] = bf2f(v.y >> 16);
@@ -306,7 +359,7 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   const size_t ap = (size_t)kM * a.nq * SK_HD;
   if (pos64 < 0 || pos64 >= a.max_len) {  // a stream past its cache: zero output, error word set
     if (split == 0) {
-      store_terms(a.att, ap, (size_t)b * a.nq * SK_HD + (2 * kvh + p) * SK_HD + d, 0.f);
+      store_terms(a.att, ap, att_index(a, b, (2 * kvh + p) * SK_HD + d), 0.f);
       if (t == 0) atomicCAS(a.err, 0, 5);
     }
     return;
@@ -437,7 +490,7 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   }
 
   if (ns == 1) {  // the whole cache in this block: the output directly, nothing to merge
-    store_terms(a.att, ap, (size_t)b * a.nq * SK_HD + (2 * kvh + p) * SK_HD + d, l > 0.f ? o / l : 0.f);
+    store_terms(a.att, ap, att_index(a, b, (2 * kvh + p) * SK_HD + d), l > 0.f ? o / l : 0.f);
     return;
   }
   // publish the partial for k_bmerge
@@ -480,7 +533,7 @@ __global__ __launch_bounds__(kThreads) void k_bmerge(AttnArgs a) {
     }
   }
   const size_t ap = (size_t)kM * a.nq * SK_HD;
-  store_terms(a.att, ap, (size_t)b * a.nq * SK_HD + (2 * kvh + p) * SK_HD + d, L > 0.f ? O / L : 0.f);
+  store_terms(a.att, ap, att_index(a, b, (2 * kvh + p) * SK_HD + d), L > 0.f ? O / L : 0.f);
 }
 
 // ---- greedy pick + embedding of the next input ---------------------------------------------------------------
@@ -551,7 +604,7 @@ __global__ __launch_bounds__(kThreads) void k_bpick(PickArgs a) {
   for (int k = t; k < a.H; k += kThreads) {
     const float v = bf2f(row[k]);
     a.h[(size_t)b * a.H + k] = v;
-    store_terms(a.xa, (size_t)kM * a.H, (size_t)b * a.H + k, v * a.nw0[k]);
+    store_terms(a.xa, (size_t)kM * a.H, plane_index<true>(b, k, a.H), v * a.nw0[k]);
     ss = __builtin_fmaf(v, v, ss);
   }
   ss = wave_sum(ss);
@@ -561,46 +614,70 @@ __global__ __launch_bounds__(kThreads) void k_bpick(PickArgs a) {
 }
 
 // ---- dispatch ------------------------------------------------------------------------------------------------
-// Launch plan: R row groups per wave (2 from N = 8192 rows up, else 1), slices of CW 64-wide chunks (8, halved while
-// the grid has fewer than kMinWg workgroups), S = K / (64 CW) slices, NB row blocks of 4 R groups. Measured on the
-// 1.7B step (16 streams): slices of 16 chunks (96 KB of LDS, fewer slices) 7657 and a minimum of 96 workgroups 7958
-// against 7992 stream-frames/s.
-constexpr int kMinWg = 192;
-struct Plan { int R, CW, S, NB; };
-Plan plan(int N, int K) {
+// Launch plan: S slices of K (one up to K = 2048, else slices of 1536 or 2048), RG row groups per workgroup (as many as
+// keep the grid near one workgroup per CU, up to 3), NW waves. Best of a sweep over 4, 8 and 16 waves, 1 to 6 groups and
+// 1 to 12 slices on the 1.7B and 0.6B shapes; what the rule's neighbours took, in us: qkv 4096 x 2048 5.8 (2 groups 6.7,
+// 2 slices 7.0), o 2048 x 2048 4.9 (2 slices 5.5), gate/up 12288 x 2048 9.0 with 16 waves and 3 groups (8 waves 10.0, 4
+// groups 9.9), down 2048 x 6144 7.2 (3 slices 7.8, 6 slices 8.0), gate/up 6144 x 1024 5.2 (1 group 6.0, 3 groups 5.8),
+// down 1024 x 3072 5.7 (6 slices and 2 groups 5.4).
+struct Plan {
+  int S, RG, NW;
+};
+Plan plan(int N, int K, bool tiled) {
   Plan pl;
-  pl.R = N >= 8192 ? 2 : 1;
-  pl.NB = (N / 16 + 4 * pl.R - 1) / (4 * pl.R);
-  pl.CW = 8;
-  while (pl.CW > 2 && (K % (64 * pl.CW) != 0 ||
-                       (pl.NB * (K / (64 * pl.CW)) < kMinWg && K / (32 * pl.CW) <= kMaxSlices)))
-    pl.CW /= 2;
-  pl.S = K / (64 * pl.CW);
+  pl.S = K <= 2048 ? 1 : K % 2048 == 0 && K % 1536 != 0 ? K / 2048 : K / 1536;
+  const int g = N / 16 * pl.S;
+  pl.RG = g <= 256 ? 1 : g <= 512 ? 2 : 3;
+  // 16 waves halve what each of three row groups' waves waits for; row-major planes would need 96 KB of LDS
+  pl.NW = tiled && pl.RG == 3 && K / pl.S % 1024 == 0 ? 16 : 8;
   return pl;
 }
 int64_t part_floats(int N, int K) {
-  const Plan pl = plan(N, K);
-  return pl.S > 1 ? (int64_t)pl.S * (N / 16) * 256 : 0;
+  const int S = plan(N, K, true).S;
+  return S > 1 ? (int64_t)S * (N / 16) * 256 : 0;
 }
-template <int OUT, int R>
-hipError_t launch_cw(const GemmArgs& p, const Plan& pl, hipStream_t st) {
-  const dim3 grid(pl.NB, pl.S);
-  switch (pl.CW) {
-    case 2: hipLaunchKernelGGL((k_bgemm<OUT, R, 2>), grid, dim3(kThreads), 0, st, p); break;
-    case 4: hipLaunchKernelGGL((k_bgemm<OUT, R, 4>), grid, dim3(kThreads), 0, st, p); break;
-    case 8: hipLaunchKernelGGL((k_bgemm<OUT, R, 8>), grid, dim3(kThreads), 0, st, p); break;
+template <int OUT, bool TILED, int NW, int RG, int KW>
+void launch_one(const GemmArgs& p, hipStream_t st) {
+  hipLaunchKernelGGL((k_bgemm<OUT, TILED, NW, RG, KW>), dim3((p.N / 16 + RG - 1) / RG, p.S), dim3(64 * NW), 0, st, p);
+}
+template <int OUT, bool TILED, int RG>
+hipError_t launch_kw(const GemmArgs& p, int NW, hipStream_t st) {
+  const int C = p.K / p.S / 64;  // chunks of a slice
+  if constexpr (TILED && RG == 3) {
+    if (NW == 16) {
+      if (C == 16) launch_one<OUT, TILED, 16, RG, 1>(p, st);
+      else launch_one<OUT, TILED, 16, RG, 2>(p, st);
+      return hipGetLastError();
+    }
+  }
+  switch (C) {
+    case 8: launch_one<OUT, TILED, 8, RG, 1>(p, st); break;
+    case 16: launch_one<OUT, TILED, 8, RG, 2>(p, st); break;
+    case 24: launch_one<OUT, TILED, 8, RG, 3>(p, st); break;
+    case 32: launch_one<OUT, TILED, 8, RG, 4>(p, st); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
 }
+template <int OUT, bool TILED>
+hipError_t launch_rg(const GemmArgs& p, const Plan& pl, hipStream_t st) {
+  switch (pl.RG) {
+    case 1: return launch_kw<OUT, TILED, 1>(p, pl.NW, st);
+    case 2: return launch_kw<OUT, TILED, 2>(p, pl.NW, st);
+    default: return launch_kw<OUT, TILED, 3>(p, pl.NW, st);
+  }
+}
 bool k_supported(int K) { return K == 512 || K == 1024 || K == 2048 || K == 3072 || K == 4096 || K == 6144; }
 
+template <bool TILED>
 hipError_t launch_gemm(GemmArgs p, int mode, hipStream_t st) {
-  const Plan pl = plan(p.N, p.K);
+  const Plan pl = plan(p.N, p.K, TILED);
   p.S = pl.S;
-  if (mode == kOutF32) return pl.R == 2 ? launch_cw<kOutF32, 2>(p, pl, st) : launch_cw<kOutF32, 1>(p, pl, st);
-  if (mode == kOutSwiglu) return pl.R == 2 ? launch_cw<kOutSwiglu, 2>(p, pl, st) : launch_cw<kOutSwiglu, 1>(p, pl, st);
-  return pl.R == 2 ? launch_cw<kOutAcc, 2>(p, pl, st) : launch_cw<kOutAcc, 1>(p, pl, st);
+  switch (mode) {
+    case kOutF32: return launch_rg<kOutF32, TILED>(p, pl, st);
+    case kOutSwiglu: return launch_rg<kOutSwiglu, TILED>(p, pl, st);
+    default: return launch_rg<kOutAcc, TILED>(p, pl, st);
+  }
 }
 
 int check_gemm(const GemmArgs& p, int mode) {
@@ -666,14 +743,13 @@ extern "C" int64_t sk_bgemm_workspace_size(int N, int K) {
 extern "C" int sk_bgemm(const void* x, const float* ssp, int np, float eps, const void* w_tiled, const uint16_t* s, int N,
                         int K, int mode, float* out, void* act, void* xn, const float* nw, float* ssp_out,
                         void* workspace, int64_t workspace_bytes, void* stream) {
-  GemmArgs p{(const bf16_t*)x, ssp, np, eps, (const uint8_t*)w_tiled, s, N, K, out, (bf16_t*)act, (bf16_t*)xn, nw, ssp_out,
-             1, nullptr, nullptr};
+  GemmArgs p{(const bf16_t*)x, ssp, np, eps, (const uint8_t*)w_tiled, s, N, K, out, (bf16_t*)act, (bf16_t*)xn, nw, ssp_out};
   if (check_gemm(p, mode)) return sk_set_error(SK_EINVAL, "sk_bgemm: bad shape, mode or pointer");
   if (!workspace || !SK_ALIGNED16(workspace)) return sk_set_error(SK_EINVAL, "sk_bgemm: workspace must be 16-byte aligned");
   if (workspace_bytes < sk_bgemm_workspace_size(N, K)) return sk_set_error(SK_EWORKSPACE, "sk_bgemm: workspace too small");
   p.part = (float*)workspace;
   p.counters = (unsigned*)((char*)workspace + up256(part_floats(N, K) * 4));
-  return sk_check_launch(launch_gemm(p, mode, (hipStream_t)stream), "sk_bgemm");
+  return sk_check_launch(launch_gemm<false>(p, mode, (hipStream_t)stream), "sk_bgemm");
 }
 
 extern "C" int sk_batch_terms(void) { return kTerms; }
@@ -738,7 +814,7 @@ extern "C" int sk_batch_attn(const float* qkv, const float* qn, const float* kn,
   char* ws = (char*)workspace;
   const int64_t part = up256(256);
   AttnArgs at{qkv, qn, kn, eps, rope, (bf16_t*)Kc, (bf16_t*)Vc, pos, max_len, nq, nkv, (bf16_t*)att,
-              (float*)(ws + part), (int*)ws};
+              (float*)(ws + part), (int*)ws, false};
   hipLaunchKernelGGL(k_battn, dim3(batch * nkv, (max_len + kAttnChunk - 1) / kAttnChunk), dim3(kThreads), 0,
                      (hipStream_t)stream, at);
   hipError_t e = hipGetLastError();
@@ -771,19 +847,19 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
   bf16_t* att = (bf16_t*)(ws + w.att);
   bf16_t* act = (bf16_t*)(ws + w.act);
   float* logits = (float*)(ws + w.logits);
+  const int nqkv = (nq + 2 * nkv) * SK_HD;
   float* gpart = (float*)(ws + w.gpart);
   unsigned* gctr = (unsigned*)(ws + w.gctr);
-  const int nqkv = (nq + 2 * nkv) * SK_HD;
   hipError_t e = hipSuccess;
   for (int l = 0; l < d->n_layers && e == hipSuccess; l++) {
     const sk_layer_desc& L = d->layers[l];
     const int np_a = l == 0 ? 1 : H / 16;
     GemmArgs g1{xa, ssa, np_a, d->eps, (const uint8_t*)L.qkv_w, L.qkv_s, nqkv, H, qkv, nullptr, nullptr, nullptr, nullptr,
                 1, gpart, gctr};
-    e = launch_gemm(g1, kOutF32, st);
+    e = launch_gemm<true>(g1, kOutF32, st);
     if (e != hipSuccess) break;
     AttnArgs at{qkv, L.qn, L.kn, d->eps, d->rope, (bf16_t*)L.kc, (bf16_t*)L.vc, d->pos, d->max_len, nq, nkv, att,
-                (float*)(ws + w.part), (int*)(ws + w.err)};
+                (float*)(ws + w.part), (int*)(ws + w.err), true};
     hipLaunchKernelGGL(k_battn, dim3(d->batch * nkv, (d->max_len + kAttnChunk - 1) / kAttnChunk), dim3(kThreads), 0, st, at);
     e = hipGetLastError();
     if (e != hipSuccess) break;
@@ -792,16 +868,16 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
     if (e != hipSuccess) break;
     GemmArgs g2{att, nullptr, 0, d->eps, (const uint8_t*)L.o_w, L.o_s, H, nq * SK_HD, h, nullptr, xb, L.post_norm, ssb,
                 1, gpart, gctr};
-    e = launch_gemm(g2, kOutAcc, st);
+    e = launch_gemm<true>(g2, kOutAcc, st);
     if (e != hipSuccess) break;
     GemmArgs g3{xb, ssb, H / 16, d->eps, (const uint8_t*)L.gu_w, L.gu_s, 2 * I, H, nullptr, act, nullptr, nullptr, nullptr,
                 1, gpart, gctr};
-    e = launch_gemm(g3, kOutSwiglu, st);
+    e = launch_gemm<true>(g3, kOutSwiglu, st);
     if (e != hipSuccess) break;
     const float* nw_next = l + 1 < d->n_layers ? d->layers[l + 1].in_norm : d->norm;
     GemmArgs g4{act, nullptr, 0, d->eps, (const uint8_t*)L.down_w, L.down_s, H, I, h, nullptr, xa, nw_next, ssa,
                 1, gpart, gctr};
-    e = launch_gemm(g4, kOutAcc, st);
+    e = launch_gemm<true>(g4, kOutAcc, st);
     if (e != hipSuccess) break;
     if (d->layer_out)
       e = hipMemcpyAsync(d->layer_out + (size_t)l * kM * H, h, (size_t)kM * H * 4, hipMemcpyDeviceToDevice, st);
@@ -809,7 +885,7 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
   if (e == hipSuccess) {
     GemmArgs gh{xa, ssa, H / 16, d->eps, (const uint8_t*)d->head_w, d->head_s, V, H, logits, nullptr, nullptr, nullptr,
                 nullptr, 1, gpart, gctr};
-    e = launch_gemm(gh, kOutF32, st);
+    e = launch_gemm<true>(gh, kOutF32, st);
   }
   if (e == hipSuccess && d->logits) e = hipMemcpyAsync(d->logits, logits, (size_t)kM * V * 4, hipMemcpyDeviceToDevice, st);
   if (e == hipSuccess) e = embed_launch(d, 1, st);

@@ -287,3 +287,66 @@ def test_batch17b_against_fixture(gpu):
     print(f"  codes equal: {int((got == ref).sum())} of {ref.size}", flush=True)
     assert np.array_equal(got, ref)
     assert rel_err(eng.logits[:16], gold["logits_last"]) < TOL
+
+
+@pytest.mark.parametrize("N,K", [(6160, 1024), (8224, 2048), (8224, 512), (1040, 4096), (1072, 6144), (2080, 3072), (16, 512)])
+def test_bgemm_row_blocks_and_slices(gpu, N, K):
+    """Row counts that leave the last workgroup's row groups short (two or three groups per workgroup) and K cut into
+    slices, called twice on one workspace (the arrival counters end at zero). Bound: the products are exact and the
+    roundings of K fp32 additions add up as a random walk, sqrt(K) 2^-24 of the sums' size, 4.7e-6 at the longest K here;
+    twice that where two such sums are multiplied or squared."""
+    from sokutou_amd.batch import tile
+    from sokutou_amd.kernels import _Lin
+
+    print(f"sk_bgemm N={N} K={K}: short row blocks, K slices", flush=True)
+    g = torch.Generator().manual_seed(N * 7 + K)
+    lin = _Lin(torch.randn(N, K, generator=g) * 0.02, "i8row")
+    lin.w, lin.s = lin.w.to(gpu), lin.s.to(gpu)
+    wt = tile(lin)
+    x, h0, nw = torch.randn(16, K, generator=g), torch.randn(16, N, generator=g), 1 + 0.1 * torch.randn(N, generator=g)
+    ref = x.double() @ lin.dequant().cpu().double().T
+    xp, nwg = _terms(x).to(gpu), nw.to(gpu)
+    p, st = _lib.ptr, _lib.stream()
+    ws = torch.zeros(int(_lib.load().sk_bgemm_workspace_size(N, K)), dtype=torch.uint8, device=gpu)
+    for rep in range(2):
+        out = torch.zeros(16, N, device=gpu)
+        _lib.call("sk_bgemm", p(xp), None, 0, 1e-6, p(wt), p(lin.s), N, K, 0, p(out), None, None, None, None, p(ws), ws.numel(), st)
+        h, xn, ss = h0.to(gpu), torch.zeros(xp.shape[0], 16, N, device=gpu, dtype=torch.bfloat16), torch.zeros(N // 16, 16, device=gpu)
+        _lib.call("sk_bgemm", p(xp), None, 0, 1e-6, p(wt), p(lin.s), N, K, 2, p(h), None, p(xn), p(nwg), p(ss), p(ws), ws.numel(), st)
+        href = h0.double() + ref
+        assert rel_err(out, ref.numpy()) < 5e-6
+        assert rel_err(h, href.numpy()) < 5e-6
+        assert rel_err(xn.float().sum(0), (href * nw.double()).numpy()) < 5e-6
+        assert rel_err(ss, href.view(16, N // 16, 16).square().sum(2).t().numpy()) < 1e-5
+        if N % 32 == 0:
+            act = torch.zeros(xp.shape[0], 16, N // 2, device=gpu, dtype=torch.bfloat16)
+            _lib.call("sk_bgemm", p(xp), None, 0, 1e-6, p(wt), p(lin.s), N, K, 1, None, p(act), None, None, None, p(ws), ws.numel(), st)
+            a, b = ref[:, 0::2], ref[:, 1::2]
+            assert rel_err(act.float().sum(0), (a * torch.sigmoid(a) * b).numpy()) < 1e-5
+
+
+@pytest.mark.parametrize("hidden,inter,nq,vocab,batch", [(1024, 3072, 16, 3072, 3), (512, 4096, 4, 528, 16), (3072, 512, 8, 1040, 1),
+                                                         (2048, 6144, 16, 8224, 2)])
+def test_batch_shapes_against_oracle(gpu, monkeypatch, hidden, inter, nq, vocab, batch):
+    """One layer and head of every supported projection length through the batched step (whose planes stay in the
+    matrix cores' order), two steps against the fp32 oracle."""
+    from oracle.workload import batch_oracle
+
+    monkeypatch.setitem(syn.SHAPES, "t", syn.TalkerShape(hidden=hidden, n_layers=1, nq=nq, nkv=nq // 2, inter=inter, vocab=vocab))
+    monkeypatch.setitem(syn.WORKLOADS, "t", dict(shape="t", n_layers=1, kv=0, batch=batch, kv_lo=3, kv_hi=300, frames=2))
+    print(f"batched step, hidden {hidden} inter {inter} nq {nq} vocab {vocab} batch {batch}", flush=True)
+    eng, T, tok = _run_small(gpu, name="t")
+    orc, oT, otok, s = batch_oracle("t", 1)
+    assert (oT, otok) == (T, tok)
+    eng.layer_out = torch.zeros((1, 16, hidden), device=gpu)
+    eng.logits = torch.zeros((16, vocab), device=gpu)
+    t, pos = list(tok), list(T)
+    for _ in range(2):
+        lo: list = []
+        t, lg = orc.step(t, pos, lo)
+        pos = [p_ + 1 for p_ in pos]
+        eng.step()
+        torch.cuda.synchronize()
+        assert eng.error() == 0
+        assert rel_err(eng.layer_out[0, :batch], lo[0]) < TIGHT and rel_err(eng.logits[:batch], lg) < TIGHT
+    assert eng.picked().cpu().numpy()[-1].tolist() == t
