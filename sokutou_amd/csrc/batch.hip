@@ -307,16 +307,23 @@ __global__ void k_tile(const int8_t* __restrict__ w, int8_t* __restrict__ tiled,
 
 // ---- ragged split-K decode attention -----------------------------------------------------------------------
 // Block (stream b, kv head g, split s) covers positions [128 s, 128 s + 128) of stream b's cache up to its current
-// position, in two passes of 64 positions whose K/V rows are all loaded at the top; the split that holds the position
-// also normalises, rotates and appends this step's K and V. Partials (max, sum, Σ p v) go to the workspace and a
-// second launch (k_bmerge, one block per (b, g)) merges them in split order and writes the attention output as bf16
-// term planes; a stream whose cache fits one split writes its output directly. The partials need no
-// device-coherent stores and no arrival counter this way (the launch boundary orders them): 22.5 against 22.9 us
-// per layer for merging in the attention launch by the last split to arrive. Numerics as sk_attn
-// (qwen3/kernels.py:338-414).
-constexpr int kPass = 64;
-constexpr int kAttnPasses = 2;
-constexpr int kAttnChunk = kPass * kAttnPasses;
+// position; the split that holds the position also normalises, rotates and appends this step's K and V. Each of its four
+// waves takes 32 positions, all of whose K and V rows are loaded at the top, and works alone to its own maximum, sum and
+// Σ p v; the four meet once in LDS. The block's partial (max, sum, Σ p v) goes to the workspace and a second launch
+// (k_bmerge, one block per (b, g)) merges the splits in order and writes the attention output as bf16 term planes; a
+// stream whose cache fits one split writes its output directly. The partials need no device-coherent stores and no
+// arrival counter this way (the launch boundary orders them). Numerics as sk_attn (qwen3/kernels.py:338-414).
+//   * Scores on the matrix cores: q of both heads is kept as kTerms bf16 terms in rows 4 head + term of the MFMA's A, so
+//     the products are exact and a lane (16 head + position) finds its score's terms in its own registers: no sum over
+//     lanes, and the softmax statistics are 16-lane DPP reductions of two values. Σ p v stays on the vector units (fp32
+//     weights, 24 instructions per four rows), where a row of V is one contiguous load.
+//   * What bounds it is the memory rate: with all arithmetic taken out it takes as long. Per call (with the merge) of 16
+//     streams of 64..2048 positions, 82 MB: 27.4 us in two passes of 64 positions with the softmax statistics and the sums
+//     over lanes shared by the block (ten barriers), 22.5 with waves alone, 20.1 (5.4 TB/s behind the launches) with
+//     nontemporal loads, 19.8 for the loads alone; 133 MB 35.8 / 31.2 / 26.6. Five streams of 8..200: 10.0 -> 7.1, one
+//     of 1500 11.5 -> 7.3, sixteen of 20..128 8.9 -> 7.0 (latency and the launches).
+constexpr int kWavePos = 32;                       // positions of one wave
+constexpr int kAttnChunk = kWavePos * kThreads / SK_WAVE;
 constexpr int kAttnSplitMax = 32;  // max_len <= 4096
 constexpr int kPart = SK_HD + 2;
 constexpr float kInvSqrtHd = 0.08838834764831845f;
@@ -345,13 +352,32 @@ __device__ __forceinline__ void unpack8(uint4 v, float* o) {
   o[4] = bf2f(v.z & 0xffffu); o[5] = bf2f(v.z >> 16); o[6] = bf2f(v.w & 0xffffu); o[7] = bf2f(v.w >> 16);
 }
 
+// Sums x over the four 16-lane rows: lane (row r, l) returns the sums of head r / 2, elements 4 (r % 2) .. + 4 of a0 / a1
+// (head 0 / 1) over the lanes l of every row.
+__device__ __forceinline__ float4 rows_sum(const float (&a0)[8], const float (&a1)[8]) {
+  float h[8], o[4];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a0[e]), __float_as_uint(a1[e]), false, false);
+    h[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[e]), __float_as_uint(h[e + 4]), false, false);
+    o[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
+  }
+  return make_float4(o[0], o[1], o[2], o[3]);
+}
+
 __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
-  __shared__ float qsh[2][SK_HD];
-  __shared__ float ksh[SK_HD];
-  __shared__ float vsh[SK_HD];
-  __shared__ float sc[2][kPass];
-  __shared__ float red[16];
-  __shared__ float opart[4][4][16][17];
+  constexpr int kWaves = kThreads / SK_WAVE;
+  static_assert(kTerms <= 4, "a head's terms fill four rows of the MFMA");
+  __shared__ __align__(16) bf16_t qt[8][SK_HD + 8];  // row 4 head + term
+  __shared__ __align__(16) bf16_t ksh[SK_HD];        // this step's K and V rows as the cache holds them
+  __shared__ __align__(16) bf16_t vsh[SK_HD];
+  __shared__ float es[kWaves][kWavePos][2];          // softmax weights of a wave's positions, both heads
+  __shared__ __align__(16) float op[kWaves][2][SK_HD];
+  __shared__ float ml[kWaves][2][2];
   const int bg = blockIdx.x, b = bg / a.nkv, kvh = bg % a.nkv, split = blockIdx.y;
   const int t = threadIdx.x, p = t >> 7, d = t & (SK_HD - 1), w = t >> 6, lane = t & 63, gq = lane >> 4, sl = lane & 15;
   const int qs = (a.nq + 2 * a.nkv) * SK_HD;
@@ -366,127 +392,122 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   }
   const int pos = (int)pos64, T = pos + 1, ns = (T + kAttnChunk - 1) / kAttnChunk;
   if (split >= ns) return;
-  const int t0 = split * kAttnChunk, n = min(kAttnChunk, T - t0), npass = (n + kPass - 1) / kPass;
-  const bool has_pos = split == ns - 1;
+  const int t0 = split * kAttnChunk, n = min(kAttnChunk, T - t0);
+  const bool has_pos = split == ns - 1;  // only this split can have fewer than kAttnChunk positions
   bf16_t* Kh = a.Kc + ((size_t)b * a.nkv + kvh) * a.max_len * SK_HD;
   bf16_t* Vh = a.Vc + ((size_t)b * a.nkv + kvh) * a.max_len * SK_HD;
-  const float* qrow = a.qkv + (size_t)b * qs;
-  // lane (w, gq, sl) holds dims [8 sl, 8 sl + 8) of positions 16 i + 4 w + gq of a pass. Every load is issued
-  // unconditionally (rows past the block's range read row t0 instead and are never used; the row at pos is taken
-  // from LDS), so all of them are in flight together.
-  auto load_pass = [&](int ps, uint4 (&kr)[4], uint4 (&vr)[4]) {
+  // this step's inputs first (the wait for them must not also wait for the cache rows): wave 0 q of head 2 g, wave 1 q of
+  // head 2 g + 1, wave 2 k, wave 3 v, dims lane and lane + 64 per lane
+  const float* src = a.qkv + (size_t)b * qs + (w < 2 ? (2 * kvh + w) * SK_HD : a.nq * SK_HD + ((w - 2) * a.nkv + kvh) * SK_HD);
+  const float* nw = w < 2 ? a.qn : a.kn;
+  const float* rp = a.rope + (size_t)pos * SK_HD;
+  const float x0 = gload(src + lane), x1 = gload(src + lane + 64), n0 = gload(nw + lane), n1 = gload(nw + lane + 64);
+  const float cs = gload(rp + lane), sn = gload(rp + lane + 64);
+  __builtin_amdgcn_sched_barrier(0);
+  // every cache row of the wave: lane (gq, sl) holds K of positions 16 i + sl, dims 32 c + 8 gq .. + 8 (the MFMA's B), and V
+  // of positions 4 i + gq, dims 8 sl .. + 8. Rows past the split's range read row t0 instead.
+  uint4 kr[2][4], vr[8];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int jj = ps * kPass + 16 * i + 4 * w + gq;
-      const size_t row = (size_t)(jj < n ? t0 + jj : t0) * SK_HD + 8 * sl;
-      kr[i] = gload4((const uint4*)(Kh + row));
-      vr[i] = gload4((const uint4*)(Vh + row));
-    }
-  };
-  // this step's inputs first (the wait for them must not also wait for the cache rows), then every cache row
-  const float c = a.rope[(size_t)pos * SK_HD + (d & 63)], s = a.rope[(size_t)pos * SK_HD + 64 + (d & 63)];
-  const float qv = qrow[(2 * kvh + p) * SK_HD + d];
-  const float kv = has_pos ? qrow[a.nq * SK_HD + p * a.nkv * SK_HD + kvh * SK_HD + d] : 0.f;
-  const float qw = a.qn[d], kw = a.kn[d];
-  uint4 kr[kAttnPasses][4], vr[kAttnPasses][4];
+  for (int i = 0; i < 2; i++) {
+    const int jj = kWavePos * w + 16 * i + sl, row = jj < n ? t0 + jj : t0;
 #pragma unroll
-  for (int ps = 0; ps < kAttnPasses; ps++) load_pass(ps, kr[ps], vr[ps]);
-  // q of both heads (and, in the split holding pos, this step's k / v): per-head RMSNorm, RoPE, bf16 append
-  {
-    const float sq = wave_sum(qv * qv), sk = wave_sum(kv * kv);
-    if (lane == 0) { red[w] = sq; red[4 + w] = sk; }
-    __syncthreads();
-    qsh[p][d] = qv * rsqrtf((red[2 * p] + red[2 * p + 1]) / SK_HD + a.eps) * qw;
-    if (has_pos) {
-      if (p == 0) ksh[d] = kv * rsqrtf((red[4] + red[5]) / SK_HD + a.eps) * kw;
-      else vsh[d] = bf2f(f2bf(kv));
-    }
-    __syncthreads();
-    const float qr = (qsh[p][d] * c + (d < 64 ? -qsh[p][d + 64] : qsh[p][d - 64]) * s) * kInvSqrtHd;
-    float krot = 0.f;
-    if (has_pos && p == 0) krot = bf2f(f2bf(ksh[d] * c + (d < 64 ? -ksh[d + 64] : ksh[d - 64]) * s));
-    __syncthreads();
-    qsh[p][d] = qr;
-    if (has_pos) {
-      if (p == 0) { ksh[d] = krot; Kh[(size_t)pos * SK_HD + d] = f2bf(krot); }
-      else Vh[(size_t)pos * SK_HD + d] = f2bf(vsh[d]);
-    }
-    __syncthreads();
+    for (int c = 0; c < 4; c++) kr[i][c] = ld_stream((const uint4*)(Kh + (uint32_t)(row * SK_HD + 32 * c + 8 * gq)));
   }
-  float q0[8], q1[8];
 #pragma unroll
-  for (int e = 0; e < 8; e++) { q0[e] = qsh[0][8 * sl + e]; q1[e] = qsh[1][8 * sl + e]; }
-  float m = -INFINITY, l = 0.f, o = 0.f;  // running partial of head p, dim d
-#pragma unroll
-  for (int ps = 0; ps < kAttnPasses; ps++) {
-    if (ps >= npass) break;  // uniform over the block
-    const int base = ps * kPass, np = min(kPass, n - base);
-    // scores of both heads
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int jl = 16 * i + 4 * w + gq;
-      float k8[8];
-      if (base + jl < n && t0 + base + jl == pos) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) k8[e] = ksh[8 * sl + e];
-      } else {
-        unpack8(kr[ps][i], k8);
-      }
-      float s0 = 0.f, s1 = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; e++) { s0 = __builtin_fmaf(q0[e], k8[e], s0); s1 = __builtin_fmaf(q1[e], k8[e], s1); }
-      s0 = row16_sum(s0);
-      s1 = row16_sum(s1);
-      if (sl == 0 && jl < np) { sc[0][jl] = s0; sc[1][jl] = s1; }
+  for (int i = 0; i < 8; i++) {
+    const int jj = kWavePos * w + 4 * i + gq, row = jj < n ? t0 + jj : t0;
+    vr[i] = ld_stream((const uint4*)(Vh + (uint32_t)(row * SK_HD + 8 * sl)));
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  if (w < 3) {  // per-head RMSNorm, RoPE
+    const float inv = rsqrtf(wave_sum(x0 * x0 + x1 * x1) / SK_HD + a.eps);
+    const float y0 = x0 * inv * n0, y1 = x1 * inv * n1;
+    const float r0 = y0 * cs + -y1 * sn, r1 = y1 * cs + y0 * sn;
+    if (w < 2) {
+      store_terms(&qt[4 * w][0], SK_HD + 8, lane, r0 * kInvSqrtHd);
+      store_terms(&qt[4 * w][0], SK_HD + 8, lane + 64, r1 * kInvSqrtHd);
+    } else if (has_pos) {
+      const bf16_t k0 = f2bf(r0), k1 = f2bf(r1);
+      ksh[lane] = k0;
+      ksh[lane + 64] = k1;
+      Kh[(size_t)pos * SK_HD + lane] = k0;
+      Kh[(size_t)pos * SK_HD + lane + 64] = k1;
     }
-    __syncthreads();
-    // pass softmax statistics per head (threads 0-127: head 0, 128-255: head 1)
-    const float sv = d < np ? sc[p][d] : -INFINITY;
-    const float mx = wave_max(sv);
-    if (lane == 0) red[8 + w] = mx;
-    __syncthreads();
-    const float mp = fmaxf(red[8 + 2 * p], red[8 + 2 * p + 1]);
-    const float ev = d < np ? expf(sv - mp) : 0.f;
-    const float se = wave_sum(ev);
-    if (d < np) sc[p][d] = ev;
-    if (lane == 0) red[12 + w] = se;
-    __syncthreads();
-    const float lp = red[12 + 2 * p] + red[12 + 2 * p + 1];
-    // Σ p_j v_j for both heads
-    float a0[8], a1[8];
+  } else if (has_pos) {
+    const bf16_t v0 = f2bf(x0), v1 = f2bf(x1);
+    vsh[lane] = v0;
+    vsh[lane + 64] = v1;
+    Vh[(size_t)pos * SK_HD + lane] = v0;
+    Vh[(size_t)pos * SK_HD + lane + 64] = v1;
+  }
+  __syncthreads();
+  if (has_pos) {  // the row at pos from LDS; zero V past it (its weight is zero, the memory may hold anything)
 #pragma unroll
-    for (int e = 0; e < 8; e++) { a0[e] = 0.f; a1[e] = 0.f; }
+    for (int i = 0; i < 2; i++)
+      if (t0 + kWavePos * w + 16 * i + sl == pos)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      const int jl = 16 * i + 4 * w + gq;
-      if (jl < np) {
-        float v8[8];
-        if (t0 + base + jl == pos) {
+        for (int c = 0; c < 4; c++) kr[i][c] = *(const uint4*)&ksh[32 * c + 8 * gq];
 #pragma unroll
-          for (int e = 0; e < 8; e++) v8[e] = vsh[8 * sl + e];
-        } else {
-          unpack8(vr[ps][i], v8);
-        }
-        const float e0 = sc[0][jl], e1 = sc[1][jl];
-#pragma unroll
-        for (int e = 0; e < 8; e++) { a0[e] = __builtin_fmaf(e0, v8[e], a0[e]); a1[e] = __builtin_fmaf(e1, v8[e], a1[e]); }
-      }
+    for (int i = 0; i < 8; i++) {
+      const int jj = kWavePos * w + 4 * i + gq;
+      if (t0 + jj == pos) vr[i] = *(const uint4*)&vsh[8 * sl];
+      else if (jj >= n) vr[i] = make_uint4(0, 0, 0, 0);
     }
+  }
+  const bool used = sl < 8 && (sl & 3) < kTerms;
+  bf16x8 qa[4];
 #pragma unroll
-    for (int e = 0; e < 8; e++) { opart[w][gq][sl][e] = a0[e]; opart[w][gq][sl][8 + e] = a1[e]; }
-    __syncthreads();
-    float op = 0.f;
+  for (int c = 0; c < 4; c++) {
+    const uint4 v = *(const uint4*)&qt[4 * ((sl >> 2) & 1) + min(sl & 3, kTerms - 1)][32 * c + 8 * gq];
+    qa[c] = as_bf16x8(used ? v : make_uint4(0, 0, 0, 0));
+  }
+  // scores: lane 16 head + sl (the lower half of the wave) holds positions sl and 16 + sl
+  float sv[2], e[2];
 #pragma unroll
-    for (int ww = 0; ww < 4; ww++)
+  for (int i = 0; i < 2; i++) {
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int gg = 0; gg < 4; gg++) op += opart[ww][gg][d >> 3][p * 8 + (d & 7)];
-    // fold the pass into the running partial
-    const float mn = fmaxf(m, mp);
-    const float fo = m == -INFINITY ? 0.f : expf(m - mn), fp = expf(mp - mn);
-    o = o * fo + op * fp;
-    l = l * fo + lp * fp;
-    m = mn;
-    __syncthreads();  // sc / opart are rewritten by the next pass
+    for (int c = 0; c < 4; c++) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[c], as_bf16x8(kr[i][c]), acc, 0, 0, 0);
+    float s = acc[kTerms - 1];
+#pragma unroll
+    for (int q = kTerms - 2; q >= 0; q--) s += acc[q];
+    sv[i] = kWavePos * w + 16 * i + sl < n ? s : -INFINITY;
+  }
+  const float mw = row16_max(fmaxf(sv[0], sv[1]));
+#pragma unroll
+  for (int i = 0; i < 2; i++) e[i] = kWavePos * w + 16 * i + sl < n ? expf(sv[i] - mw) : 0.f;
+  const float lw = row16_sum(e[0] + e[1]);
+  if (gq < 2) {
+    es[w][sl][gq] = e[0];
+    es[w][16 + sl][gq] = e[1];
+    if (sl == 0) {
+      ml[w][gq][0] = mw;
+      ml[w][gq][1] = lw;
+    }
+  }
+  wave_sync();
+  float a0[8], a1[8];
+#pragma unroll
+  for (int k = 0; k < 8; k++) { a0[k] = 0.f; a1[k] = 0.f; }
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const float2 ew = *(const float2*)&es[w][4 * i + gq][0];
+    float v8[8];
+    unpack8(vr[i], v8);
+#pragma unroll
+    for (int k = 0; k < 8; k++) { a0[k] = __builtin_fmaf(ew.x, v8[k], a0[k]); a1[k] = __builtin_fmaf(ew.y, v8[k], a1[k]); }
+  }
+  *(float4*)&op[w][gq >> 1][8 * sl + 4 * (gq & 1)] = rows_sum(a0, a1);
+  __syncthreads();
+  // the waves' partials of head p, dim d
+  float m = ml[0][p][0], l = 0.f, o = 0.f;
+#pragma unroll
+  for (int q = 1; q < kWaves; q++) m = fmaxf(m, ml[q][p][0]);
+#pragma unroll
+  for (int q = 0; q < kWaves; q++) {
+    const float f = ml[q][p][0] == -INFINITY ? 0.f : expf(ml[q][p][0] - m);
+    l = __builtin_fmaf(f, ml[q][p][1], l);
+    o = __builtin_fmaf(f, op[q][p][d], o);
   }
 
   if (ns == 1) {  // the whole cache in this block: the output directly, nothing to merge
@@ -499,37 +520,53 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   pp[2 + d] = o;
 }
 
-// Block (stream b, kv head g): the log-sum-exp merge of k_battn's partials of (b, g) in split order (thread (p, d): q
-// head 2 g + p, dim d), written as bf16 term planes. Streams past their cache and streams of one split were handled
-// by k_battn.
+// Block (stream b, kv head g): the log-sum-exp merge of k_battn's partials of (b, g) (thread (p, d): q head 2 g + p, dim
+// d), written as bf16 term planes. Streams past their cache and streams of one split were handled by k_battn. Bound by
+// the launch and one memory round trip: the partials of every split that the cache could have are loaded together with
+// the position, those past it are not used, and one wave finds the splits' weights for all.
 __global__ __launch_bounds__(kThreads) void k_bmerge(AttnArgs a) {
-  __shared__ float mls[2][kAttnSplitMax][2];
+  static_assert(2 * kAttnSplitMax == SK_WAVE, "one lane per head and split");
+  __shared__ __align__(16) float fs[2][kAttnSplitMax];  // a split's weight, negative where it has none
+  __shared__ float ls[2];
   const int bg = blockIdx.x, b = bg / a.nkv, kvh = bg % a.nkv;
   const int t = threadIdx.x, p = t >> 7, d = t & (SK_HD - 1);
+  const int nmax = (a.max_len + kAttnChunk - 1) / kAttnChunk;  // at most kAttnSplitMax
+  const int cc = t % kAttnSplitMax;
+  const float2 st = *(const float2*)(a.part + (bg * 2 * kAttnSplitMax + t % SK_WAVE) * kPart);
+  float oc[kAttnSplitMax];
+  const float* po = a.part + (bg * 2 + p) * kAttnSplitMax * kPart + 2 + d;
+#pragma unroll
+  for (int k0 = 0; k0 < kAttnSplitMax; k0 += 8)
+    if (k0 < nmax)
+#pragma unroll
+      for (int k = k0; k < k0 + 8; k++) oc[k] = gload(po + k * kPart);
   const int64_t pos64 = a.pos[b];
   if (pos64 < 0 || pos64 >= a.max_len) return;
   const int ns = ((int)pos64 + kAttnChunk) / kAttnChunk;
   if (ns == 1) return;
-  if (t < 2 * ns) {
-    const int pp = t / ns, cc = t % ns;
-    const float* q = a.part + ((bg * 2 + pp) * kAttnSplitMax + cc) * kPart;
-    mls[pp][cc][0] = q[0];
-    mls[pp][cc][1] = q[1];
+  if (t < SK_WAVE) {  // lane 32 head + split
+    const float m = cc < ns ? st.x : -INFINITY;
+    const float r = row16_max(m);
+    const float ma = fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 0)), __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 16)));
+    const float mb = fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 32)), __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 48)));
+    const bool has = cc < ns && m != -INFINITY;
+    const float f = has ? expf(m - (t < kAttnSplitMax ? ma : mb)) : -1.f;
+    fs[t / kAttnSplitMax][cc] = f;
+    const float q = row16_sum(has ? f * st.y : 0.f);
+    const float la = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 0)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 16));
+    const float lb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 32)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 48));
+    if (t < 2) ls[t] = t ? lb : la;
   }
-  float oc[kAttnSplitMax];
-  const float* po = a.part + (bg * 2 + p) * kAttnSplitMax * kPart + 2 + d;
-#pragma unroll
-  for (int k = 0; k < kAttnSplitMax; k++) oc[k] = po[(k < ns ? k : 0) * kPart];
   __syncthreads();
-  float M = -INFINITY;
-  for (int cc = 0; cc < ns; cc++) M = fmaxf(M, mls[p][cc][0]);
-  float L = 0.f, O = 0.f;
+  const float L = ls[p];
+  float O = 0.f;
 #pragma unroll
-  for (int k = 0; k < kAttnSplitMax; k++) {
-    if (k < ns && mls[p][k][0] != -INFINITY) {
-      const float f = expf(mls[p][k][0] - M);
-      L = __builtin_fmaf(f, mls[p][k][1], L);
-      O = __builtin_fmaf(f, oc[k], O);
+  for (int k0 = 0; k0 < kAttnSplitMax; k0 += 8) {
+    if (k0 >= ns) break;
+#pragma unroll
+    for (int k = k0; k < k0 + 8; k++) {
+      const float f = fs[p][k], x = __builtin_fmaf(f, oc[k], O);
+      O = f < 0.f ? O : x;
     }
   }
   const size_t ap = (size_t)kM * a.nq * SK_HD;

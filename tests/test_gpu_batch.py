@@ -350,3 +350,41 @@ def test_batch_shapes_against_oracle(gpu, monkeypatch, hidden, inter, nq, vocab,
         assert eng.error() == 0
         assert rel_err(eng.layer_out[0, :batch], lo[0]) < TIGHT and rel_err(eng.logits[:batch], lg) < TIGHT
     assert eng.picked().cpu().numpy()[-1].tolist() == t
+
+
+@pytest.mark.parametrize("pos", [[0, 15, 16, 31, 32, 33, 47, 48], [63, 64, 95, 96, 97, 126, 127, 128], [159, 160, 255, 256, 1151, 1152, 1343, 1344],
+                                 [4095]])
+def test_batch_attention_at_wave_boundaries(gpu, pos):
+    """sk_batch_attn with streams that end on either side of a wave's 32 positions and of its 16-position score tiles, up to
+    the longest cache; rows past a stream's position hold NaN, and so do the workspace's partials before the call. Bound:
+    each score is a sum of 3 x 128 exact products and each output one of up to 4096, fp32 roundings that add up as a random
+    walk, sqrt(4096) 2^-24 = 3.8e-6 of the largest value, and the weights' exponentials a few 2^-24 more; and one in a few
+    thousand of this step's keys falls on the other side of a bf16 rounding, which moves a one-position softmax not at all
+    and a score of the rest by 2^-9 of one of 128 products, 2e-5 of a weight."""
+    nkv, nq, max_len = 2, 4, max(pos) + 1
+    B = len(pos)
+    print(f"sk_batch_attn: streams at positions {pos}, NaN beyond", flush=True)
+    rng = np.random.default_rng(pos[0] + 1)
+    qkv = np.zeros((16, (nq + 2 * nkv) * 128), np.float32)
+    qkv[:B] = rng.standard_normal((B, qkv.shape[1])).astype(np.float32)
+    qn, kn = ((1 + 0.1 * rng.standard_normal(128)).astype(np.float32) for _ in range(2))
+    Kc, Vc = (O.bf16_round(rng.standard_normal((B, nkv, max_len, 128)).astype(np.float32)) for _ in range(2))
+    rope = O.rope_table(syn.inv_freq(syn.shape("1.7b")), max_len)
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a)).to(gpu)
+    Kg, Vg = dev(Kc).to(torch.bfloat16), dev(Vc).to(torch.bfloat16)
+    for b, q in enumerate(pos):
+        Kg[b, :, q:] = float("nan")
+        Vg[b, :, q:] = float("nan")
+    L, p = _lib.load(), _lib.ptr
+    att = torch.zeros((int(L.sk_batch_terms()), 16, nq * 128), dtype=torch.bfloat16, device=gpu)
+    ws = torch.full((int(L.sk_batch_attn_workspace_size(nkv)),), 255, dtype=torch.uint8, device=gpu)
+    ws[:256] = 0
+    posg, qkvg, qng, kng, ropeg = torch.tensor(pos, dtype=torch.int64, device=gpu), dev(qkv), dev(qn), dev(kn), dev(rope)
+    _lib.call("sk_batch_attn", p(qkvg), p(qng), p(kng), 1e-6, p(ropeg), p(Kg), p(Vg), p(posg), B, max_len, nq, nkv,
+              p(att), p(ws), ws.numel(), _lib.stream())
+    torch.cuda.synchronize()
+    assert int(ws[:4].view(torch.int32).item()) == 0
+    got = att.float().sum(0).cpu().numpy()
+    for b, q in enumerate(pos):
+        ref = O.attention(qkv[b], qn, kn, 1e-6, rope, Kc[b].copy(), Vc[b].copy(), q, nq, nkv, cache_bf16=True)
+        assert rel_err(got[b], ref) < 2e-5, (b, q)
