@@ -64,6 +64,37 @@ def test_gemv_family(gpu, wd, N, K):
         assert rel_err(out, O.rms_gemv(x, nw, 1e-6, deq, swiglu=True)) < 1e-5
 
 
+@pytest.mark.parametrize("wd", ["i8row", "i8g32", "bf16", "f32"])
+@pytest.mark.parametrize("N,K", [(2, 512), (5, 1536), (2047, 1536), (2049, 2560), (3, 4096), (8200, 512), (8195, 2560), (2050, 7680), (1028, 8192)])
+def test_gemv_row_blocks_and_steps(gpu, wd, N, K):
+    """The workgroup's edges: rows that leave its last groups short at one, two and four rows per group, input lengths whose
+    steps do not divide among the waves, more steps than the waves hold at once, and the longest input. Bound: K fp32
+    roundings that add up as a random walk, sqrt(8192) 2^-24 = 5.4e-6 of the largest output's terms."""
+    print(f"gemv wd={wd} N={N} K={K}: row blocks and steps", flush=True)
+    rng = np.random.default_rng(N * 3 + K)
+    w = (rng.standard_normal((N, K)) * 0.02).astype(F32)
+    _, _, deq = O.quantize(w, wd)
+    lin = _Lin(_t(w, gpu), wd)
+    x, nw = rng.standard_normal(K).astype(F32), (1 + 0.1 * rng.standard_normal(K)).astype(F32)
+    bias, base = rng.standard_normal(N).astype(F32), rng.standard_normal(N).astype(F32)
+    p, st, code = _lib.ptr, _lib.stream(), _lib.WD[wd]
+    xg, nwg, bg = _t(x, gpu), _t(nw, gpu), _t(bias, gpu)
+    d64, x64 = deq.astype(np.float64), x.astype(np.float64)
+    inv = 1 / np.sqrt(np.mean(x64 * x64) + 1e-6)
+    out = _t(base, gpu)
+    _lib.call("sk_gemv", p(xg), p(lin.w), p(lin.s), p(bg), p(out), N, K, 1, code, 1, st)
+    assert rel_err(out, d64 @ x64 + bias + base) < 1e-5
+    out = torch.full((N + 4,), 7.0, device=gpu)
+    _lib.call("sk_rms_gemv", p(xg), p(nwg), 1e-6, p(lin.w), p(lin.s), p(out), N, K, 0, code, 1, st)
+    y = d64 @ (x64 * nw) * inv
+    assert rel_err(out[:N], y) < 1e-5 and bool((out[N:] == 7).all())
+    if N % 2 == 0:
+        out = torch.full((N // 2 + 4,), 7.0, device=gpu)
+        _lib.call("sk_rms_gemv", p(xg), p(nwg), 1e-6, p(lin.w), p(lin.s), p(out), N, K, 1, code, 1, st)
+        ref = y[0::2] / (1 + np.exp(-y[0::2])) * y[1::2]
+        assert rel_err(out[: N // 2], ref) < 1e-5 and bool((out[N // 2:] == 7).all())
+
+
 def _attn_case(gpu, seed, nkv, max_len, pos, ct):
     nq = 2 * nkv
     rng = np.random.default_rng(seed)
