@@ -26,8 +26,6 @@
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 constexpr int kM = 16;         // rows of every activation buffer (streams)
@@ -53,30 +51,16 @@ __device__ __forceinline__ bf16x8 i8x8_bf16(uint32_t a, uint32_t b) {
   r.w = pack_hi16((float)(int8_t)(b >> 16), (float)(int8_t)(b >> 24));
   return __builtin_bit_cast(bf16x8, r);
 }
-__device__ __forceinline__ uint4 gload4(const uint4* p) {
-  const u32x4 v = *(gptr<const u32x4>)p;
-  return make_uint4(v.x, v.y, v.z, v.w);
-}
-__device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
-  u32x4 r = {v.x, v.y, v.z, v.w};
-  return __builtin_bit_cast(bf16x8, r);
-}
 // v as kTerms bf16 terms written to planes [kTerms][plane] at index i
 __device__ __forceinline__ void store_terms(bf16_t* __restrict__ planes, size_t plane, size_t i, float v) {
 #pragma unroll
   for (int t = 0; t < kTerms; t++) {
-    const bf16_t b = f2bf(v);
+    const bf16_t b = f2bf_hw(v);
     planes[t * plane + i] = b;
     v -= bf2f(b);
   }
 }
 
-// Orders this wave's LDS stores before its later loads of the same words by other lanes (LDS operations of one wave
-// complete in order, so no wait or barrier is needed).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
 // rotation (in fours) of staging segment s = 2 (j & 1) + h, s = 0..3
 __device__ __forceinline__ int sq_rot(int s) { return 2 * ((s >> 1) & 1) + (s & 1); }
 
@@ -347,28 +331,6 @@ __device__ __forceinline__ size_t att_index(const AttnArgs& a, int b, int k) {
   return a.tiled ? plane_index<true>(b, k, a.nq * SK_HD) : plane_index<false>(b, k, a.nq * SK_HD);
 }
 
-__device__ __forceinline__ void unpack8(uint4 v, float* o) {
-  o[0] = bf2f(v.x & 0xffffu); o[1] = bf2f(v.x >> 16); o[2] = bf2f(v.y & 0xffffu); o[3] = bf2f(v.y >> 16);
-  o[4] = bf2f(v.z & 0xffffu); o[5] = bf2f(v.z >> 16); o[6] = bf2f(v.w & 0xffffu); o[7] = bf2f(v.w >> 16);
-}
-
-// Sums x over the four 16-lane rows: lane (row r, l) returns the sums of head r / 2, elements 4 (r % 2) .. + 4 of a0 / a1
-// (head 0 / 1) over the lanes l of every row.
-__device__ __forceinline__ float4 rows_sum(const float (&a0)[8], const float (&a1)[8]) {
-  float h[8], o[4];
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a0[e]), __float_as_uint(a1[e]), false, false);
-    h[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
-  }
-#pragma unroll
-  for (int e = 0; e < 4; e++) {
-    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[e]), __float_as_uint(h[e + 4]), false, false);
-    o[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
-  }
-  return make_float4(o[0], o[1], o[2], o[3]);
-}
-
 __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   constexpr int kWaves = kThreads / SK_WAVE;
   static_assert(kTerms <= 4, "a head's terms fill four rows of the MFMA");
@@ -493,7 +455,7 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   for (int i = 0; i < 8; i++) {
     const float2 ew = *(const float2*)&es[w][4 * i + gq][0];
     float v8[8];
-    unpack8(vr[i], v8);
+    unpack_bf8(vr[i], v8);
 #pragma unroll
     for (int k = 0; k < 8; k++) { a0[k] = __builtin_fmaf(ew.x, v8[k], a0[k]); a1[k] = __builtin_fmaf(ew.y, v8[k], a1[k]); }
   }
@@ -547,14 +509,14 @@ __global__ __launch_bounds__(kThreads) void k_bmerge(AttnArgs a) {
   if (t < SK_WAVE) {  // lane 32 head + split
     const float m = cc < ns ? st.x : -INFINITY;
     const float r = row16_max(m);
-    const float ma = fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 0)), __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 16)));
-    const float mb = fmaxf(__int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 32)), __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r), 48)));
+    const float ma = fmaxf(lane_value(r, 0), lane_value(r, 16));
+    const float mb = fmaxf(lane_value(r, 32), lane_value(r, 48));
     const bool has = cc < ns && m != -INFINITY;
     const float f = has ? expf(m - (t < kAttnSplitMax ? ma : mb)) : -1.f;
     fs[t / kAttnSplitMax][cc] = f;
     const float q = row16_sum(has ? f * st.y : 0.f);
-    const float la = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 0)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 16));
-    const float lb = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 32)) + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(q), 48));
+    const float la = lane_value(q, 0) + lane_value(q, 16);
+    const float lb = lane_value(q, 32) + lane_value(q, 48);
     if (t < 2) ls[t] = t ? lb : la;
   }
   __syncthreads();

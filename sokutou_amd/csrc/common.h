@@ -23,6 +23,8 @@ __device__ __forceinline__ bf16_t f2bf(float f) {
   u += 0x7fffu + ((u >> 16) & 1u);
   return (bf16_t)(u >> 16);
 }
+// The same rounding in one instruction; a NaN keeps its sign and payload bits (for terms that stay inside a kernel's sums).
+__device__ __forceinline__ bf16_t f2bf_hw(float f) { return __builtin_bit_cast(bf16_t, (__bf16)f); }
 __device__ __forceinline__ float h2f(uint16_t h) {
   _Float16 x;
   __builtin_memcpy(&x, &h, 2);
@@ -189,6 +191,48 @@ __device__ __forceinline__ float buf_ldf(const void* base, uint32_t off) {
 template <int POL = kPolDev>
 __device__ __forceinline__ void buf_stf(void* base, uint32_t off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), make_rsrc(base), off, 0, POL);
+}
+
+// ---- matrix-core operands and wave-local exchange -----------------------------------------------------------------
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(4))) float f32x4;
+__device__ __forceinline__ bf16x8 as_bf16x8(uint4 v) {
+  uint32_t r __attribute__((ext_vector_type(4))) = {v.x, v.y, v.z, v.w};
+  return __builtin_bit_cast(bf16x8, r);
+}
+__device__ __forceinline__ uint4 gload4(const uint4* p) {
+  uint32_t v __attribute__((ext_vector_type(4))) = *(gptr<const uint32_t __attribute__((ext_vector_type(4)))>)p;
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+// 8 bf16 as floats
+__device__ __forceinline__ void unpack_bf8(uint4 v, float* o) {
+  o[0] = bf2f(v.x & 0xffffu); o[1] = bf2f(v.x >> 16); o[2] = bf2f(v.y & 0xffffu); o[3] = bf2f(v.y >> 16);
+  o[4] = bf2f(v.z & 0xffffu); o[5] = bf2f(v.z >> 16); o[6] = bf2f(v.w & 0xffffu); o[7] = bf2f(v.w >> 16);
+}
+// Orders this wave's LDS stores before its later loads of the same words by other lanes (LDS operations of one wave
+// complete in order, so no wait or barrier is needed).
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+// Sums over the four 16-lane rows: lane (row r, l) returns the sums of a0 (r < 2) or a1, elements 4 (r % 2) .. + 4, over the
+// lanes l of every row.
+__device__ __forceinline__ float4 rows_sum(const float (&a0)[8], const float (&a1)[8]) {
+  float h[8], o[4];
+#pragma unroll
+  for (int e = 0; e < 8; e++) {
+    const auto v = __builtin_amdgcn_permlane32_swap(__float_as_uint(a0[e]), __float_as_uint(a1[e]), false, false);
+    h[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const auto v = __builtin_amdgcn_permlane16_swap(__float_as_uint(h[e]), __float_as_uint(h[e + 4]), false, false);
+    o[e] = __uint_as_float(v[0]) + __uint_as_float(v[1]);
+  }
+  return make_float4(o[0], o[1], o[2], o[3]);
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {  // lane: uniform
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // ---- sampled picks ---------------------------------------------------------------------------------------------

@@ -25,13 +25,6 @@ namespace {
 constexpr int kGroups = 4;  // 16-lane row groups per wave
 constexpr int kStep = 256;  // inputs a wave takes at a time: one float4 per lane
 
-// Orders this wave's LDS stores before its later loads of the same words by other lanes (LDS operations of one wave
-// complete in order, so no wait or barrier is needed).
-__device__ __forceinline__ void wave_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-}
-
 template <int POL>
 __device__ __forceinline__ uint4 ldw(const uint4* p) {
   if constexpr (POL == 1) return ld_stream(p);

@@ -150,6 +150,41 @@ def test_attention(gpu, ct, nkv, max_len, pos):
     assert int(ws[4 : 4 + 4 * nkv].view(torch.int32).abs().sum()) == 0
 
 
+@pytest.mark.parametrize("ct", ["bf16", "f32"])
+@pytest.mark.parametrize("max_len,pos", [(33, 31), (64, 63), (65, 64), (128, 127), (129, 31), (300, 128), (1024, 1023), (1025, 1024), (2048, 127),
+                                         (2049, 2048), (4097, 255), (4097, 256), (4097, 4096), (9000, 8999)])
+def test_attention_plans_and_unwritten_rows(gpu, ct, max_len, pos):
+    """Both sides of every change of the split plan (waves per block, blocks, passes) and of a wave's rows, with NaN in every
+    cache row at or past the position and in the workspace's partials, which is one sized for a longer cache and was
+    last used by it. Bound as above: fp32 sums of 128 products and of up to 9000 weighted rows."""
+    print(f"attn ct={ct} max_len={max_len} pos={pos}: NaN beyond the position", flush=True)
+    nkv, nq = 2, 4
+    rng = np.random.default_rng(max_len + pos)
+    qkv = rng.standard_normal((nq + 2 * nkv) * 128).astype(F32)
+    qn, kn = ((1 + 0.1 * rng.standard_normal(128)).astype(F32) for _ in range(2))
+    Kc, Vc = (rng.standard_normal((nkv, max_len, 128)).astype(F32) for _ in range(2))
+    if ct == "bf16":
+        Kc, Vc = O.bf16_round(Kc), O.bf16_round(Vc)
+    rope = O.rope_table(syn.inv_freq(syn.shape("0.6b")), max_len)
+    dt = torch.bfloat16 if ct == "bf16" else torch.float32
+    Kg, Vg = _t(Kc, gpu).to(dt), _t(Vc, gpu).to(dt)
+    Kg[:, pos:] = float("nan")
+    Vg[:, pos:] = float("nan")
+    L, p = _lib.load(), _lib.ptr
+    ws = torch.full((int(L.sk_attn_workspace_size(nq, nkv, 9000)),), 255, dtype=torch.uint8, device=gpu)
+    ws[:256] = 0
+    out, posg = torch.zeros(nq * 128, device=gpu), torch.tensor([pos], dtype=torch.int64, device=gpu)
+    qkvg, qng, kng, ropeg = _t(qkv, gpu), _t(qn, gpu), _t(kn, gpu), _t(rope, gpu)
+    for _ in range(2):
+        _lib.call("sk_attn", p(qkvg), p(qng), p(kng), 1e-6, p(ropeg), p(Kg), p(Vg), p(posg), 0, max_len, nq, nkv, p(out), p(ws), ws.numel(),
+                  _lib.CT[ct], _lib.stream())
+    torch.cuda.synchronize()
+    assert int(ws[:256].view(torch.int32).abs().sum()) == 0  # no error, counters back at zero
+    ref = O.attention(qkv, qn, kn, 1e-6, rope, Kc.copy(), Vc.copy(), pos, nq, nkv, cache_bf16=(ct == "bf16"))
+    assert rel_err(out, ref) < 2e-5
+    assert bool(torch.isnan(Kg[:, pos + 1:]).all()) and bool(torch.isfinite(Kg[:, pos]).all())
+
+
 def test_attention_invalid_position_sets_error_word(gpu):
     nkv, max_len = 8, 64
     rng = np.random.default_rng(5)
