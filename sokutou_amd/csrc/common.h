@@ -193,6 +193,24 @@ __device__ __forceinline__ void buf_stf(void* base, uint32_t off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), make_rsrc(base), off, 0, POL);
 }
 
+template <int CTRL, int ROW_MASK = 0xf, int BANK_MASK = 0xf>
+__device__ __forceinline__ uint32_t dpp_u(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, BANK_MASK, false);
+}
+__device__ __forceinline__ uint32_t row16_umax(uint32_t v) {
+  v = max(v, dpp_u<0xB1>(v));   // quad_perm [1,0,3,2]
+  v = max(v, dpp_u<0x4E>(v));   // quad_perm [2,3,0,1]
+  v = max(v, dpp_u<0x124>(v));  // row_ror:4
+  v = max(v, dpp_u<0x128>(v));  // row_ror:8
+  return v;
+}
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v) {  // uniform result
+  v = row16_umax(v);
+  const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+  const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)v, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
+  return max(max(a, b), max(c, d));
+}
+
 // ---- matrix-core operands and wave-local exchange -----------------------------------------------------------------
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;

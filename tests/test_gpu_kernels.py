@@ -218,7 +218,7 @@ def test_attention_invalid_position_sets_error_word(gpu):
 
 def test_rmsnorm_embed(gpu):
     rng = np.random.default_rng(9)
-    for K in (1024, 2048, 100):
+    for K in (1024, 2048, 100, 1, 1025, 3000, 4096, 6145):
         h = rng.standard_normal(K).astype(F32)
         nw = (1 + 0.1 * rng.standard_normal(K)).astype(F32)
         out = torch.zeros(K, device=gpu)
@@ -364,6 +364,38 @@ def test_sampled_picks_match_oracle(gpu):
     print(f"  {n} draws: {n - len(bad) - ties} identical, {ties} within rounding of a tie", flush=True)
     assert not bad, bad[:5]
     assert ties <= 2
+
+
+@pytest.mark.parametrize("top_k", [2, 50, 63, 64, 65, 255, 256, 257])
+def test_sampled_picks_at_the_path_boundaries(gpu, top_k):
+    """The ranked pick (top_k up to 64, up to 256 candidates), its fallback (more candidates, fewer entries than top_k) and the
+    bisected paths: ordinary values, all equal, ten finite ones, values in a few steps (many ties) and NaNs, at
+    vocabularies around the group and block sizes. Picks equal the oracle's (whole values)."""
+    from sokutou_amd.sampler import FusedSampler
+
+    fs = FusedSampler(gpu)
+    fs.set_seed(99)
+    rng = np.random.default_rng(top_k)
+    out, draw, ties = torch.zeros(1, dtype=torch.int64, device=gpu), 0, 0
+    for V in (16, 65, 256, 257, 300, 1025, 2048, 4095, 4096):
+        for kind in ("normal", "equal", "few", "steps", "nan"):
+            lg = (rng.standard_normal(V) * 2).astype(F32)
+            if kind == "equal":
+                lg[:] = -1.5
+            elif kind == "few":
+                lg[rng.permutation(V)[10:]] = -np.inf
+            elif kind == "steps":
+                lg = np.round(lg * 2) / 2
+            elif kind == "nan":
+                lg[rng.integers(0, V, V // 4)] = np.nan
+            fs(_t(lg.astype(F32), gpu), out, True, 0.9, top_k)
+            torch.cuda.synchronize()
+            ref, g = O.sample_draw(lg.astype(F32), float(np.float32(1.0 / 0.9)), top_k, 99, draw, exact=True)
+            draw += 1
+            if int(out) != ref:
+                assert _near_tie(g, int(out), ref), (V, kind, int(out), ref)
+                ties += 1
+    assert int(fs.counter) == draw and ties <= 1
 
 
 def test_sampled_pick_replays_from_a_graph(gpu):
