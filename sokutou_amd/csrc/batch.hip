@@ -554,62 +554,75 @@ struct PickArgs {
   int* err;
 };
 
-__global__ __launch_bounds__(kThreads) void k_bpick(PickArgs a) {
-  __shared__ float bv[kThreads];
-  __shared__ int bi[kThreads];
-  __shared__ float red[kThreads / SK_WAVE];
-  __shared__ int id_s;
-  const int b = blockIdx.x, t = threadIdx.x;
+// Bound by the launch and two dependent memory round trips (the logits, then the embedding row of the pick): 1024 threads
+// with four logits each in flight and the largest found by DPP maxima: 10.9 -> 4.3 us per step of 16 streams (V 3072, H 2048)
+// against 256 threads that took twelve logits one after the other and met in eight LDS steps.
+constexpr int kPickThreads = 1024, kPickPer = 4;
+__global__ __launch_bounds__(kPickThreads) void k_bpick(PickArgs a) {
+  constexpr int kWaves = kPickThreads / SK_WAVE;
+  static_assert(kWaves == 16, "one wave's result per lane of a row");
+  __shared__ uint32_t wkey[kWaves], widx[kWaves];
+  __shared__ float red[kWaves];
+  const int b = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
+  int id;
   if (a.pick) {
     const float* lg = a.logits + (size_t)b * a.V;
-    float best = 0.f;
-    int bidx = -1;
-    for (int k = t; k < a.V; k += kThreads) {
-      const float v = lg[k];
-      if (v == v && (bidx < 0 || v > best)) { best = v; bidx = k; }
-    }
-    bv[t] = best;
-    bi[t] = bidx;
-    __syncthreads();
-    for (int s = kThreads / 2; s > 0; s >>= 1) {
-      if (t < s) {
-        const int j2 = bi[t + s];
-        if (j2 >= 0 && (bi[t] < 0 || bv[t + s] > bv[t] || (bv[t + s] == bv[t] && j2 < bi[t]))) {
-          bv[t] = bv[t + s];
-          bi[t] = j2;
-        }
+    const int64_t f = a.nstep[b], pos = a.pos[b];
+    uint32_t best = 0, bi = 0xffffffffu;  // key 0 is below every value's
+    for (int k0 = 0; k0 < a.V; k0 += kPickThreads * kPickPer) {
+      float v[kPickPer];
+#pragma unroll
+      for (int j = 0; j < kPickPer; j++) v[j] = gload(lg + min(k0 + j * kPickThreads + t, a.V - 1));
+#pragma unroll
+      for (int j = 0; j < kPickPer; j++) {
+        const int k = k0 + j * kPickThreads + t;
+        const uint32_t key = k < a.V && v[j] == v[j] ? order_key(v[j] == 0.f ? 0.f : v[j]) : 0u;  // -0 equals +0, NaN never wins
+        if (key > best) { best = key; bi = (uint32_t)k; }
       }
-      __syncthreads();
     }
+    const uint32_t top = wave_umax(best);
+    const uint32_t ti = ~wave_umax(best == top ? ~bi : 0u);
+    if (lane == 0) { wkey[w] = top; widx[w] = ti; }
+    __syncthreads();
+    const uint32_t k2 = wkey[lane & 15], tk = wave_umax(k2);  // every wave finds the pick
+    const uint32_t pick = ~wave_umax(k2 == tk ? ~widx[lane & 15] : 0u);
+    id = pick >= (uint32_t)a.V ? 0 : (int)pick;
     if (t == 0) {
-      const int id = bi[0] < 0 ? 0 : bi[0];
-      id_s = id;
       a.ids[b] = id;
-      const int64_t f = a.nstep[b];
       if (f >= 0 && f < a.max_frames) a.codes[f * kM + b] = id;
       else atomicCAS(a.err, 0, 6);
       a.nstep[b] = f + 1;
-      a.pos[b] = a.pos[b] + 1;
+      a.pos[b] = pos + 1;
     }
-  } else if (t == 0) {
-    int64_t id = a.ids[b];
-    if (id < 0 || id >= a.V) { atomicCAS(a.err, 0, 5); id = 0; }
-    id_s = (int)id;
+  } else {
+    const int64_t i = a.ids[b];
+    if (t == 0 && (i < 0 || i >= a.V)) atomicCAS(a.err, 0, 5);
+    id = i < 0 || i >= a.V ? 0 : (int)i;
   }
-  __syncthreads();
-  const int id = id_s;
   const bf16_t* row = a.emb + (size_t)id * a.H;
   float ss = 0.f;
-  for (int k = t; k < a.H; k += kThreads) {
-    const float v = bf2f(row[k]);
-    a.h[(size_t)b * a.H + k] = v;
-    store_terms(a.xa, (size_t)kM * a.H, plane_index<true>(b, k, a.H), v * a.nw0[k]);
-    ss = __builtin_fmaf(v, v, ss);
+  for (int k0 = 0; k0 < a.H; k0 += 2 * kPickThreads) {
+    float v[2], nv[2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int k = min(k0 + j * kPickThreads + t, a.H - 1);
+      v[j] = bf2f(gload(row + k));
+      nv[j] = gload(a.nw0 + k);
+    }
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+      const int k = k0 + j * kPickThreads + t;
+      if (k >= a.H) break;
+      a.h[(size_t)b * a.H + k] = v[j];
+      store_terms(a.xa, (size_t)kM * a.H, plane_index<true>(b, k, a.H), v[j] * nv[j]);
+      ss = __builtin_fmaf(v[j], v[j], ss);
+    }
   }
   ss = wave_sum(ss);
-  if ((t & 63) == 0) red[t >> 6] = ss;
+  if (lane == 0) red[w] = ss;
   __syncthreads();
-  if (t == 0) a.ssa[b] = (red[0] + red[1]) + (red[2] + red[3]);
+  const float tot = row16_sum(red[lane & 15]);
+  if (t == 0) a.ssa[b] = tot;
 }
 
 // ---- dispatch ------------------------------------------------------------------------------------------------
@@ -790,7 +803,7 @@ hipError_t embed_launch(const sk_batch_desc* d, int pick, hipStream_t st) {
   PickArgs a{(const float*)(ws + w.logits), d->vocab, d->hidden, pick, d->max_frames, d->ids, d->pos, d->codes, d->nstep,
              (const bf16_t*)d->emb, d->layers[0].in_norm, (float*)(ws + w.h), (bf16_t*)(ws + w.xa), (float*)(ws + w.ssa),
              (int*)(ws + w.err)};
-  hipLaunchKernelGGL(k_bpick, dim3(d->batch), dim3(kThreads), 0, st, a);
+  hipLaunchKernelGGL(k_bpick, dim3(d->batch), dim3(kPickThreads), 0, st, a);
   return hipGetLastError();
 }
 }  // namespace
