@@ -307,7 +307,7 @@ __global__ void k_tile(const int8_t* __restrict__ w, int8_t* __restrict__ tiled,
 //     nontemporal loads, 19.8 for the loads alone; 133 MB 35.8 / 31.2 / 26.6. Five streams of 8..200: 10.0 -> 7.1, one
 //     of 1500 11.5 -> 7.3, sixteen of 20..128 8.9 -> 7.0 (latency and the launches).
 constexpr int kWavePos = 32;                       // positions of one wave
-constexpr int kAttnChunk = kWavePos * kThreads / SK_WAVE;
+constexpr int kAttnChunk = kWavePos * 4;           // positions of a split where a cache has several (four waves)
 constexpr int kAttnSplitMax = 32;  // max_len <= 4096
 constexpr int kPart = SK_HD + 2;
 constexpr float kInvSqrtHd = 0.08838834764831845f;
@@ -331,8 +331,9 @@ __device__ __forceinline__ size_t att_index(const AttnArgs& a, int b, int k) {
   return a.tiled ? plane_index<true>(b, k, a.nq * SK_HD) : plane_index<false>(b, k, a.nq * SK_HD);
 }
 
-__global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
-  constexpr int kWaves = kThreads / SK_WAVE;
+template <int kWaves>
+__global__ __launch_bounds__(SK_WAVE * kWaves) void k_battn(AttnArgs a) {
+  constexpr int kChunk = kWavePos * kWaves;
   static_assert(kTerms <= 4, "a head's terms fill four rows of the MFMA");
   __shared__ __align__(16) bf16_t qt[8][SK_HD + 8];  // row 4 head + term
   __shared__ __align__(16) bf16_t ksh[SK_HD];        // this step's K and V rows as the cache holds them
@@ -341,27 +342,28 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   __shared__ __align__(16) float op[kWaves][2][SK_HD];
   __shared__ float ml[kWaves][2][2];
   const int bg = blockIdx.x, b = bg / a.nkv, kvh = bg % a.nkv, split = blockIdx.y;
-  const int t = threadIdx.x, p = t >> 7, d = t & (SK_HD - 1), w = t >> 6, lane = t & 63, gq = lane >> 4, sl = lane & 15;
+  const int t = threadIdx.x, p = (t >> 7) & 1, d = t & (SK_HD - 1), w = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, gq = lane >> 4, sl = lane & 15;
   const int qs = (a.nq + 2 * a.nkv) * SK_HD;
   const int64_t pos64 = a.pos[b];
   const size_t ap = (size_t)kM * a.nq * SK_HD;
   if (pos64 < 0 || pos64 >= a.max_len) {  // a stream past its cache: zero output, error word set
-    if (split == 0) {
+    if (split == 0 && t < 2 * SK_HD) {
       store_terms(a.att, ap, att_index(a, b, (2 * kvh + p) * SK_HD + d), 0.f);
       if (t == 0) atomicCAS(a.err, 0, 5);
     }
     return;
   }
-  const int pos = (int)pos64, T = pos + 1, ns = (T + kAttnChunk - 1) / kAttnChunk;
+  const int pos = (int)pos64, T = pos + 1, ns = (T + kChunk - 1) / kChunk;
   if (split >= ns) return;
-  const int t0 = split * kAttnChunk, n = min(kAttnChunk, T - t0);
-  const bool has_pos = split == ns - 1;  // only this split can have fewer than kAttnChunk positions
+  const int t0 = split * kChunk, n = min(kChunk, T - t0);
+  const bool has_pos = split == ns - 1;  // only this split can have fewer than kChunk positions
   bf16_t* Kh = a.Kc + ((size_t)b * a.nkv + kvh) * a.max_len * SK_HD;
   bf16_t* Vh = a.Vc + ((size_t)b * a.nkv + kvh) * a.max_len * SK_HD;
   // this step's inputs first (the wait for them must not also wait for the cache rows): wave 0 q of head 2 g, wave 1 q of
   // head 2 g + 1, wave 2 k, wave 3 v, dims lane and lane + 64 per lane
-  const float* src = a.qkv + (size_t)b * qs + (w < 2 ? (2 * kvh + w) * SK_HD : a.nq * SK_HD + ((w - 2) * a.nkv + kvh) * SK_HD);
-  const float* nw = w < 2 ? a.qn : a.kn;
+  const int wq = w & 3;
+  const float* src = a.qkv + (size_t)b * qs + (wq < 2 ? (2 * kvh + wq) * SK_HD : a.nq * SK_HD + ((wq - 2) * a.nkv + kvh) * SK_HD);
+  const float* nw = wq < 2 ? a.qn : a.kn;
   const float* rp = a.rope + (size_t)pos * SK_HD;
   const float x0 = gload(src + lane), x1 = gload(src + lane + 64), n0 = gload(nw + lane), n1 = gload(nw + lane + 64);
   const float cs = gload(rp + lane), sn = gload(rp + lane + 64);
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
       Kh[(size_t)pos * SK_HD + lane] = k0;
       Kh[(size_t)pos * SK_HD + lane + 64] = k1;
     }
-  } else if (has_pos) {
+  } else if (w == 3 && has_pos) {
     const bf16_t v0 = f2bf(x0), v1 = f2bf(x1);
     vsh[lane] = v0;
     vsh[lane + 64] = v1;
@@ -461,6 +463,7 @@ __global__ __launch_bounds__(kThreads) void k_battn(AttnArgs a) {
   }
   *(float4*)&op[w][gq >> 1][8 * sl + 4 * (gq & 1)] = rows_sum(a0, a1);
   __syncthreads();
+  if (t >= 2 * SK_HD) return;
   // the waves' partials of head p, dim d
   float m = ml[0][p][0], l = 0.f, o = 0.f;
 #pragma unroll
@@ -692,6 +695,25 @@ hipError_t launch_gemm(GemmArgs p, int mode, hipStream_t st) {
   }
 }
 
+// The attention of the batch: one block per stream and head that holds the whole cache up to 256 positions (eight waves,
+// four up to 128), else splits of 128 positions and the merge. Five streams in caches of 205: 6.9 us per call with two
+// splits, 6.5 in one block without the merge's launch; one block of sixteen waves up to 512 positions took 12.3 against 9.8 with
+// splits (sixteen streams), since one CU then loads what four had.
+hipError_t launch_attn(const AttnArgs& a, int batch, hipStream_t st) {
+  const int bh = batch * a.nkv;
+  if (a.max_len <= kWavePos * 4) {
+    hipLaunchKernelGGL(k_battn<4>, dim3(bh), dim3(SK_WAVE * 4), 0, st, a);
+  } else if (a.max_len <= kWavePos * 8) {
+    hipLaunchKernelGGL(k_battn<8>, dim3(bh), dim3(SK_WAVE * 8), 0, st, a);
+  } else {
+    hipLaunchKernelGGL(k_battn<4>, dim3(bh, (a.max_len + kAttnChunk - 1) / kAttnChunk), dim3(SK_WAVE * 4), 0, st, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_bmerge, dim3(bh), dim3(kThreads), 0, st, a);
+  }
+  return hipGetLastError();
+}
+
 int check_gemm(const GemmArgs& p, int mode) {
   if (!p.x || !p.w || !p.s || (!p.out && mode != kOutSwiglu)) return SK_EINVAL;
   if (p.N <= 0 || p.N % 16 || !k_supported(p.K)) return SK_EINVAL;
@@ -827,14 +849,7 @@ extern "C" int sk_batch_attn(const float* qkv, const float* qn, const float* kn,
   const int64_t part = up256(256);
   AttnArgs at{qkv, qn, kn, eps, rope, (bf16_t*)Kc, (bf16_t*)Vc, pos, max_len, nq, nkv, (bf16_t*)att,
               (float*)(ws + part), (int*)ws, false};
-  hipLaunchKernelGGL(k_battn, dim3(batch * nkv, (max_len + kAttnChunk - 1) / kAttnChunk), dim3(kThreads), 0,
-                     (hipStream_t)stream, at);
-  hipError_t e = hipGetLastError();
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_bmerge, dim3(batch * nkv), dim3(kThreads), 0, (hipStream_t)stream, at);
-    e = hipGetLastError();
-  }
-  return sk_check_launch(e, "sk_batch_attn");
+  return sk_check_launch(launch_attn(at, batch, (hipStream_t)stream), "sk_batch_attn");
 }
 
 extern "C" int sk_batch_embed(const sk_batch_desc* d, void* stream) {
@@ -872,11 +887,7 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
     if (e != hipSuccess) break;
     AttnArgs at{qkv, L.qn, L.kn, d->eps, d->rope, (bf16_t*)L.kc, (bf16_t*)L.vc, d->pos, d->max_len, nq, nkv, att,
                 (float*)(ws + w.part), (int*)(ws + w.err), true};
-    hipLaunchKernelGGL(k_battn, dim3(d->batch * nkv, (d->max_len + kAttnChunk - 1) / kAttnChunk), dim3(kThreads), 0, st, at);
-    e = hipGetLastError();
-    if (e != hipSuccess) break;
-    hipLaunchKernelGGL(k_bmerge, dim3(d->batch * nkv), dim3(kThreads), 0, st, at);
-    e = hipGetLastError();
+    e = launch_attn(at, d->batch, st);
     if (e != hipSuccess) break;
     GemmArgs g2{att, nullptr, 0, d->eps, (const uint8_t*)L.o_w, L.o_s, H, nq * SK_HD, h, nullptr, xb, L.post_norm, ssb,
                 1, gpart, gctr};

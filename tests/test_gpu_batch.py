@@ -353,7 +353,7 @@ def test_batch_shapes_against_oracle(gpu, monkeypatch, hidden, inter, nq, vocab,
 
 
 @pytest.mark.parametrize("pos", [[0, 15, 16, 31, 32, 33, 47, 48], [63, 64, 95, 96, 97, 126, 127, 128], [159, 160, 255, 256, 1151, 1152, 1343, 1344],
-                                 [4095]])
+                                 [127, 3], [255, 128, 130, 0], [256, 200], [4095]])
 def test_batch_attention_at_wave_boundaries(gpu, pos):
     """sk_batch_attn with streams that end on either side of a wave's 32 positions and of its 16-position score tiles, up to
     the longest cache; rows past a stream's position hold NaN, and so do the workspace's partials before the call. Bound:
