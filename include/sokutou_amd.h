@@ -367,6 +367,33 @@ int sk_batch_embed(const sk_batch_desc* desc, void* stream);
  * 6 n_layers + 2 launches. */
 int sk_batch_frame(const sk_batch_desc* desc, void* stream);
 
+/* ---- prompt prefill -------------------------------------------------------------------------------------------
+ * A layer's bf16 weights as the checkpoint holds them (row-major [out][in], norms [hidden] / [128]) and its cache. */
+typedef struct sk_prefill_layer {
+  const void *q, *k, *v, *o, *gate, *up, *down;
+  const void *in_norm, *post_norm, *qn, *kn;
+  void *kc, *vc;              /* bf16 [nkv][max_len][128] */
+} sk_prefill_layer;
+
+typedef struct sk_prefill_desc {
+  int n_layers, hidden, inter, nq, nkv, rows, max_len;
+  float eps;
+  const sk_prefill_layer* layers; /* host array, read during the call */
+  const void* embeds;         /* bf16 [rows][hidden] */
+  const void* norm;           /* bf16 [hidden] */
+  const float* rope;          /* [>= rows][cos 64 | sin 64] */
+  void* out;                  /* bf16 [rows][hidden]: the last hidden states after the final norm */
+  void* workspace;
+  int64_t workspace_bytes;
+} sk_prefill_desc;
+
+/* Workspace bytes of a prompt of `rows` rows (0: shape not supported); its contents need no preparation. */
+int64_t sk_prefill_workspace_size(int hidden, int inter, int nq, int nkv, int rows);
+
+/* The prompt's rows 0 .. rows - 1 through the layers (positions 0 .. rows - 1, causal), their keys and values into the
+ * caches, and the final norm. hidden, inter and nq * 128 multiples of 1024, nq == 2 nkv. 6 n_layers + 2 launches. */
+int sk_prefill(const sk_prefill_desc* desc, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -82,6 +82,20 @@ class SkBatchDesc(ctypes.Structure):
                 ("workspace_bytes", c_int64)]
 
 
+class SkPrefillLayer(ctypes.Structure):
+    """Mirror of ``sk_prefill_layer`` (include/sokutou_amd.h)."""
+    _fields_ = [(k, c_void_p) for k in ("q", "k", "v", "o", "gate", "up", "down", "in_norm", "post_norm", "qn", "kn", "kc", "vc")]
+
+
+class SkPrefillDesc(ctypes.Structure):
+    """Mirror of ``sk_prefill_desc`` (include/sokutou_amd.h)."""
+    _fields_ = [(k, c_int) for k in ("n_layers", "hidden", "inter", "nq", "nkv", "rows", "max_len")] + [
+        ("eps", c_float), ("layers", c_void_p), ("embeds", c_void_p), ("norm", c_void_p), ("rope", c_void_p), ("out", c_void_p),
+        ("workspace", c_void_p), ("workspace_bytes", c_int64)]
+
+
+_SIGS["sk_prefill_workspace_size"] = (c_int64, [c_int] * 5)
+_SIGS["sk_prefill"] = (c_int, [ctypes.POINTER(SkPrefillDesc), _P])
 _SIGS["sk_batch_terms"] = (c_int, [])
 _SIGS["sk_tile_weights"] = (c_int, [_P, _P, c_int, c_int, _P])
 _SIGS["sk_bgemm"] = (c_int, [_P, _P, c_int, c_float, _P, _P, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, c_int64, _P])

@@ -118,7 +118,7 @@ class Qwen3Fast:
         self.stats: dict = {}
         self.graphs = graphs and dev.type == "cuda"
         self.tcache = None  # the talker's KV cache as a transformers cache object (set by an engine that has one)
-        self._pf: dict = {}   # prompt length -> (graph, input buffer, positions)
+        self._pf: dict = {}   # prompt length -> (graph, input buffer, positions, and what else the graph reads)
         self._dec: dict = {}  # decode bucket -> (graph, code buffer, output)
         self._pool = torch.cuda.graph_pool_handle() if self.graphs else None
 
@@ -223,7 +223,7 @@ class Qwen3Fast:
             return
         if L not in self._pf:
             self._pf[L] = self._capture_prefill(L)
-        g, buf, _ = self._pf[L]
+        g, buf = self._pf[L][:2]
         buf.copy_(embeds)
         g.replay()
 

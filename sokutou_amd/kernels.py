@@ -66,13 +66,15 @@ def _engine_kv_cache(config, max_len: int, kc: torch.Tensor, vc: torch.Tensor):
 
     class _EngineCache(StaticCache):
         def seek(self, pos: int = 0) -> None:
-            for layer in self.layers:
-                layer.cumulative_length.fill_(int(pos))
+            self.lengths.fill_(int(pos))
 
     cache = _EngineCache(config=config, max_cache_len=max_len)
     if len(cache.layers) != kc.shape[0]:
         raise ValueError(f"the talker config has {len(cache.layers)} layers, the engine's cache {kc.shape[0]}")
     cache.layers = [_ViewLayer(kc[i], vc[i]) for i in range(kc.shape[0])]
+    cache.lengths = torch.zeros(kc.shape[0], dtype=torch.long, device=kc.device)  # one fill sets every layer's
+    for layer, n in zip(cache.layers, cache.lengths.unbind(0)):
+        layer.cumulative_length = n
     return cache
 
 
@@ -432,6 +434,7 @@ class Qwen3Kernels(Qwen3Fast):
         hf_cfg = getattr(getattr(self.talker, "model", None), "config", None)
         self.tcache = (_engine_kv_cache(hf_cfg, max_cache, self.kc, self.vc)
                        if hasattr(hf_cfg, "get_text_config") and callable(self.talker.model) else None)
+        self._prefill_own = None  # while a prefill is recorded: the prompt on the package's own kernels, if they take it
         nbytes = int(L.sk_attn_workspace_size(P.nq, P.nkv, max_cache))
         self.attn_ws = torch.zeros(nbytes, dtype=torch.uint8, device=dev)
         self.trace: list[torch.Tensor] | None = None
@@ -777,7 +780,7 @@ class Qwen3Kernels(Qwen3Fast):
         work only, so it can be recorded in a graph."""
         self.seen.zero_()
         self.ngen.zero_()
-        hidden = self._prefill_run(embeds, cpos)
+        hidden = (self._prefill_own or self._prefill_run)(embeds, cpos)
         first = _sample(self._process(self._head_logits(hidden)), self.s.do_sample, self.s.temperature, self.s.top_k)
         self.id0.copy_(first)
         self.next_id0.copy_(first)
@@ -785,6 +788,23 @@ class Qwen3Kernels(Qwen3Fast):
         self.seen.scatter_(1, first, True)
         self.ngen.fill_(1)
         self.pos.fill_(int(embeds.shape[1]))
+
+    def _capture_prefill(self, L: int):
+        """Records the prompt on the package's own kernels where they take the talker's modules and agree with them on a
+        random prompt of this length (``prefill.plan``, ``prefill.agrees``), else through the modules."""
+        from . import prefill
+
+        pre = prefill.plan(self.talker.model, self.T, self.kc, self.vc, L)
+        if pre is not None and prefill.agrees(pre, self._prefill_run, self.kc, self.vc):
+            def own(embeds, cpos):
+                self.tcache.seek(L)  # where the modules leave it
+                return pre(embeds)
+
+            self._prefill_own = own
+        try:
+            return (*super()._capture_prefill(L)[:3], pre)
+        finally:
+            self._prefill_own = None
 
     def _head_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """fp32 (1, V) codec-head logits of the last position of ``hidden`` through the talker's own module."""
