@@ -45,25 +45,24 @@ struct PGemm {
   float* ssp_out;          // kAcc: [N / 16][Mp]
 };
 
-// Workgroup (column group, row block): 16 output columns (16 of gate and of up) for MT tiles of 16 rows. Its eight waves split
-// K (kC chunks of 32 in flight each), and their sums meet in LDS.
-template <int OUT, int MT>
+// Workgroup (column block, row block): CG groups of 16 output columns (16 of gate and of up each) for MT tiles of 16 rows. Its
+// eight waves split K (kC chunks of 32 in flight each), and their sums meet in LDS.
+template <int OUT, int MT, int CG>
 __global__ __launch_bounds__(kGemmThreads) void k_pgemm(PGemm p) {
-  constexpr int RG = OUT == kSwiglu ? 2 : 1, kStrips = MT * RG * 4;
+  constexpr int kMat = OUT == kSwiglu ? 2 : 1, RG = CG * kMat, kStrips = MT * RG * 4;  // weight group r: columns r / kMat, matrix r % kMat
   __shared__ float red[kWaves][kStrips][64];
   __shared__ float ssq[kGemmThreads / (16 * MT)][16 * MT];
   __shared__ float inv_s[16 * MT];
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, nl = lane & 15, j = lane >> 4;
-  const int g = blockIdx.x, m0 = blockIdx.y * 16 * MT, C = p.K >> 5;
+  const int g = blockIdx.x * CG, m0 = blockIdx.y * 16 * MT, C = p.K >> 5;
   const bf16_t* wr[RG];
-  if constexpr (OUT == kQkv) {
-    int r = g * 16;
-    const bf16_t* b = p.w[0];
-    if (r >= p.rows[0]) { r -= p.rows[0]; b = p.w[1]; if (r >= p.rows[1]) { r -= p.rows[1]; b = p.w[2]; } }
-    wr[0] = b + (size_t)(r + nl) * p.K + 8 * j;
-  } else {
 #pragma unroll
-    for (int r = 0; r < RG; r++) wr[r] = p.w[r] + (size_t)(g * 16 + nl) * p.K + 8 * j;
+  for (int r = 0; r < RG; r++) {
+    int row = (g + r / kMat) * 16;
+    const bf16_t* b = p.w[r % kMat];
+    if constexpr (OUT == kQkv)
+      if (row >= p.rows[0]) { row -= p.rows[0]; b = p.w[1]; if (row >= p.rows[1]) { row -= p.rows[1]; b = p.w[2]; } }
+    wr[r] = b + (size_t)(row + nl) * p.K + 8 * j;
   }
   const bf16_t* xr = p.x + (size_t)(m0 >> 4) * C * 512 + lane * 8;
   f32x4 acc[MT][RG];
@@ -95,16 +94,15 @@ __global__ __launch_bounds__(kGemmThreads) void k_pgemm(PGemm p) {
           acc[m][r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(xq[c][m]), as_bf16x8(wq[c][r]), acc[m][r], 0, 0, 0);
   };
   const int per = C / kWaves;  // a multiple of kC
-  const int n = g * 16 + nl;
-  constexpr int kOwn = (MT * 4 + kWaves - 1) / kWaves;  // output strips of a wave
+  constexpr int kOut = MT * CG * 4, kOwn = (kOut + kWaves - 1) / kWaves;  // output strips (4 (CG m + c) + i), of a wave
   float hv[kOwn];
-  uint32_t nv = 0;
+  uint32_t nv[kOwn];
   if constexpr (OUT == kAcc) {  // what the epilogue needs
-    nv = gload(p.nw + n);
 #pragma unroll
     for (int o = 0; o < kOwn; o++) {
-      const int st = min(w + o * kWaves, MT * 4 - 1);
-      hv[o] = gload(p.out + (size_t)(m0 + 16 * (st >> 2) + 4 * j + (st & 3)) * p.N + n);
+      const int st = min(w + o * kWaves, kOut - 1), n = (g + (st >> 2) % CG) * 16 + nl;
+      nv[o] = gload(p.nw + n);
+      hv[o] = gload(p.out + (size_t)(m0 + 16 * ((st >> 2) / CG) + 4 * j + (st & 3)) * p.N + n);
     }
   }
   constexpr int kSs = 8, kSg = kGemmThreads / kRows;
@@ -127,7 +125,7 @@ __global__ __launch_bounds__(kGemmThreads) void k_pgemm(PGemm p) {
 #pragma unroll
     for (int r = 0; r < RG; r++)
 #pragma unroll
-      for (int i = 0; i < 4; i++) red[w][(m * 4 + i) * RG + r][lane] = acc[m][r][i];
+      for (int i = 0; i < 4; i++) red[w][((m * CG + r / kMat) * 4 + i) * kMat + r % kMat][lane] = acc[m][r][i];
   __syncthreads();
   if (p.ssp && tid < kRows) {
     float s = 0.f;
@@ -138,14 +136,14 @@ __global__ __launch_bounds__(kGemmThreads) void k_pgemm(PGemm p) {
 #pragma unroll
   for (int o = 0; o < kOwn; o++) {
     const int st = w + o * kWaves;
-    if (st >= MT * 4) break;
-    const int ml = 16 * (st >> 2) + 4 * j + (st & 3), m = m0 + ml;
+    if (st >= kOut) break;
+    const int ml = 16 * ((st >> 2) / CG) + 4 * j + (st & 3), m = m0 + ml, gc = g + (st >> 2) % CG, n = gc * 16 + nl;
     const float inv = p.ssp ? inv_s[ml] : 1.f;
     float y = 0.f, u = 0.f;
 #pragma unroll
     for (int q = 0; q < kWaves; q++) {
-      y += red[q][st * RG][lane];
-      if constexpr (RG == 2) u += red[q][st * RG + 1][lane];
+      y += red[q][st * kMat][lane];
+      if constexpr (kMat == 2) u += red[q][st * kMat + 1][lane];
     }
     if constexpr (OUT == kQkv) {
       p.out[(size_t)m * p.N + n] = y * inv;
@@ -154,9 +152,9 @@ __global__ __launch_bounds__(kGemmThreads) void k_pgemm(PGemm p) {
     } else {
       const float h = hv[o] + y;
       p.out[(size_t)m * p.N + n] = h;
-      p.xo[frag_index(m, n, p.N)] = f2bf(h * bf2f(nv));
+      p.xo[frag_index(m, n, p.N)] = f2bf(h * bf2f(nv[o]));
       const float ss = row16_sum(h * h);
-      if (nl == 0) p.ssp_out[(size_t)g * p.Mp + m] = ss;
+      if (nl == 0) p.ssp_out[(size_t)gc * p.Mp + m] = ss;
     }
   }
 }
@@ -360,20 +358,36 @@ bool shape_ok(int H, int I, int nq, int nkv, int L) {
   return H > 0 && I > 0 && nkv > 0 && nq == 2 * nkv && nkv % 2 == 0 && L > 0 && L <= 65536 && H % 1024 == 0 && I % 1024 == 0 && nq * SK_HD % 1024 == 0;
 }
 
-// Rows per workgroup: as many 16-row tiles as the prompt has, up to four, where the columns alone make a grid of 128 or more
-// workgroups; else one, so that o and down (64 column groups at 1024 columns) still fill the chip.
+// The tile of a workgroup: the largest of 4 x 4, 4 x 2, 4 x 1 (16-row tiles x column groups; gate/up's groups are two
+// matrices wide, so up to 4 x 2), fewer rows for shorter prompts, that leaves kMinWg workgroups: large tiles read the rows and
+// weights fewer times from the caches, small ones fill the chip. Against one column group everywhere, four row tiles where a row
+// of workgroups has 128 and one elsewhere (whole prompts, us): 0.6B four layers 250 rows 446 -> 389, two layers 1900 rows
+// 1152 -> 912; 1.7B two layers 33 rows 273 -> 255, 250 rows 447 -> 382, 900 rows 1140 -> 931.
+constexpr int kMinWg = 192;
+template <int OUT, int MT, int CG>
+hipError_t run(const PGemm& p, int tiles, hipStream_t st) {
+  hipLaunchKernelGGL((k_pgemm<OUT, MT, CG>), dim3(p.N / 16 / CG, (tiles + MT - 1) / MT), dim3(kGemmThreads), 0, st, p);
+  return hipGetLastError();
+}
 template <int OUT>
 hipError_t go(const PGemm& p, hipStream_t st) {
   const int tiles = (p.M + 15) / 16, G = p.N / 16;
-  const int mt = G < 128 ? 1 : tiles < 4 ? tiles : 4;
-  const dim3 grid(G, (tiles + mt - 1) / mt), th(kGemmThreads);
-  switch (mt) {
-    case 1: hipLaunchKernelGGL((k_pgemm<OUT, 1>), grid, th, 0, st, p); break;
-    case 2: hipLaunchKernelGGL((k_pgemm<OUT, 2>), grid, th, 0, st, p); break;
-    case 3: hipLaunchKernelGGL((k_pgemm<OUT, 3>), grid, th, 0, st, p); break;
-    default: hipLaunchKernelGGL((k_pgemm<OUT, 4>), grid, th, 0, st, p); break;
+  auto wgs = [&](int mt, int cg) { return (tiles + mt - 1) / mt * (G / cg); };
+  if constexpr (OUT != kSwiglu)
+    if (tiles > 3 && wgs(4, 4) >= kMinWg) return run<OUT, 4, 4>(p, tiles, st);
+  if (tiles > 3) {
+    if (wgs(4, 2) >= kMinWg) return run<OUT, 4, 2>(p, tiles, st);
+    if (wgs(4, 1) >= kMinWg) return run<OUT, 4, 1>(p, tiles, st);
   }
-  return hipGetLastError();
+  if (tiles == 3) {
+    if (wgs(3, 2) >= kMinWg) return run<OUT, 3, 2>(p, tiles, st);
+    if (wgs(3, 1) >= kMinWg) return run<OUT, 3, 1>(p, tiles, st);
+  }
+  if (tiles >= 2) {
+    if (wgs(2, 2) >= kMinWg) return run<OUT, 2, 2>(p, tiles, st);
+    if (wgs(2, 1) >= kMinWg) return run<OUT, 2, 1>(p, tiles, st);
+  }
+  return run<OUT, 1, 1>(p, tiles, st);
 }
 
 }  // namespace

@@ -46,10 +46,10 @@ class Prefill:
 
 
 # Rows times hidden size up to which the package's kernels are the faster ones: their products read each weight again for
-# every 64 rows, from the caches, where the library's large tiles catch up. Against the modules (2 layers, us): 0.6B 17 rows
-# 195 : 674, 250 rows (4 layers) 446 : 1446, 900 rows 613 : 1178, 1900 rows 1152 : 1602; 1.7B 33 rows 273 : 772, 900 rows
-# 1140 : 1336, 1900 rows 2162 : 1933.
-MAX_WORK = 1 << 21
+# every 64 rows, from the caches, where the library's large tiles catch up. Against the modules (us, two layers): 0.6B 17 rows
+# 195 : 674, 1900 rows 912 : 1609, 4000 rows 2169 : 3369; 1.7B 33 rows 255 : 777, 900 rows 931 : 1340, 2000 rows
+# 1849 : 1999.
+MAX_WORK = 1 << 22
 
 
 def _hooked(model) -> bool:

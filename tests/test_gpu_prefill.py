@@ -48,7 +48,8 @@ def _rel(a, b) -> float:
 
 
 @pytest.mark.parametrize("hidden,inter,nq,L", [(1024, 3072, 16, n) for n in (1, 2, 15, 16, 17, 32, 33, 45, 63, 64, 65, 130)] +
-                         [(2048, 1024, 8, 31), (2048, 6144, 16, 70), (1024, 1024, 8, 200)])
+                         [(2048, 1024, 8, 31), (2048, 6144, 16, 70), (1024, 1024, 8, 200), (1024, 1024, 8, 500),
+                                                     (2048, 1024, 16, 260)])
 def test_prefill_against_float64(gpu, hidden, inter, nq, L):
     """Rows on both sides of every tile (16), key tile (32) and row block (64). Inputs of each product are rounded to bf16
     (2^-9 each), so an output is off by about 2^-9 sqrt(number of roundings on its way): 6 per layer and 2 layers, 7e-3,
@@ -86,9 +87,9 @@ def test_prefill_takes_only_plain_bf16_modules(gpu):
     P = _Stack(m, "bf16", 40)
     go = lambda **kw: prefill.plan(kw.get("model", m), P, kw.get("kc", kc), kw.get("kc", kc).clone(), kw.get("rows", 9))
     assert go() is not None
-    wide = torch.zeros((1, 8, 2100, HD), dtype=torch.bfloat16, device=gpu)
-    P.rope = torch.zeros((2100, HD), device=gpu)
-    assert go(kc=wide, rows=2048) is not None and go(kc=wide, rows=2049) is None  # the library's from there on
+    wide = torch.zeros((1, 8, 4100, HD), dtype=torch.bfloat16, device=gpu)
+    P.rope = torch.zeros((4100, HD), device=gpu)
+    assert go(kc=wide, rows=4096) is not None and go(kc=wide, rows=4097) is None  # the library's from there on
     assert go(rows=41) is None and go(kc=kc.float()) is None
     assert go(model=syn.hf_talker_model(3, s).to(gpu)) is None  # fp32 weights
     m.train()
