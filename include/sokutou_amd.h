@@ -364,7 +364,7 @@ int sk_batch_embed(const sk_batch_desc* desc, void* stream);
 /* One decode step for every stream: n_layers x (qkv GEMM, ragged split-K attention with KV append at pos[b] and
  * its merge, o GEMM, gate/up GEMM, down GEMM), final RMSNorm + head GEMM, greedy pick per stream (lowest index on
  * ties), then codes / ids / nstep / pos advance and the picked rows are embedded for the next step.
- * 6 n_layers + 2 launches. */
+ * 6 n_layers + 2 launches; 5 n_layers + 2 for caches of up to 256 positions, whose attention needs no merge. */
 int sk_batch_frame(const sk_batch_desc* desc, void* stream);
 
 /* ---- prompt prefill -------------------------------------------------------------------------------------------

@@ -819,10 +819,10 @@ int check_batch(const sk_batch_desc* d) {
   return SK_OK;
 }
 
-hipError_t embed_launch(const sk_batch_desc* d, int pick, hipStream_t st) {
+hipError_t embed_launch(const sk_batch_desc* d, int pick, const float* logits, hipStream_t st) {
   char* ws = (char*)d->workspace;
   const Ws w = ws_layout(d->hidden, d->inter, d->nq, d->nkv, d->vocab);
-  PickArgs a{(const float*)(ws + w.logits), d->vocab, d->hidden, pick, d->max_frames, d->ids, d->pos, d->codes, d->nstep,
+  PickArgs a{logits, d->vocab, d->hidden, pick, d->max_frames, d->ids, d->pos, d->codes, d->nstep,
              (const bf16_t*)d->emb, d->layers[0].in_norm, (float*)(ws + w.h), (bf16_t*)(ws + w.xa), (float*)(ws + w.ssa),
              (int*)(ws + w.err)};
   hipLaunchKernelGGL(k_bpick, dim3(d->batch), dim3(kPickThreads), 0, st, a);
@@ -855,7 +855,7 @@ extern "C" int sk_batch_attn(const float* qkv, const float* qn, const float* kn,
 extern "C" int sk_batch_embed(const sk_batch_desc* d, void* stream) {
   int rc = check_batch(d);
   if (rc) return rc;
-  return sk_check_launch(embed_launch(d, 0, (hipStream_t)stream), "sk_batch_embed");
+  return sk_check_launch(embed_launch(d, 0, nullptr, (hipStream_t)stream), "sk_batch_embed");
 }
 
 extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
@@ -873,7 +873,7 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
   float* qkv = (float*)(ws + w.qkv);
   bf16_t* att = (bf16_t*)(ws + w.att);
   bf16_t* act = (bf16_t*)(ws + w.act);
-  float* logits = (float*)(ws + w.logits);
+  float* logits = d->logits ? d->logits : (float*)(ws + w.logits);  // the caller's buffer directly: no copy behind the head
   const int nqkv = (nq + 2 * nkv) * SK_HD;
   float* gpart = (float*)(ws + w.gpart);
   unsigned* gctr = (unsigned*)(ws + w.gctr);
@@ -910,7 +910,6 @@ extern "C" int sk_batch_frame(const sk_batch_desc* d, void* stream) {
                 nullptr, 1, gpart, gctr};
     e = launch_gemm<true>(gh, kOutF32, st);
   }
-  if (e == hipSuccess && d->logits) e = hipMemcpyAsync(d->logits, logits, (size_t)kM * V * 4, hipMemcpyDeviceToDevice, st);
-  if (e == hipSuccess) e = embed_launch(d, 1, st);
+  if (e == hipSuccess) e = embed_launch(d, 1, logits, st);
   return sk_check_launch(e, "sk_batch_frame");
 }
