@@ -161,8 +161,9 @@ __global__ __launch_bounds__(SK_WAVE * NW) void k_attn(const float* __restrict__
   // what does not depend on the position: wave 0 takes q of head 2 kvh, wave 1 q of head 2 kvh + 1, wave 2 k, wave 3 v, dims
   // lane and lane + 64 per lane; then every cache row of the first pass (rows past the cache's end read its last row and,
   // like rows at or past the position, are never used)
-  // (the position by a vector load ahead of all others: a scalar one would be waited for with the arguments)
-  const int64_t pv = __hip_atomic_load(pos_ptr ? pos_ptr : (const int64_t*)qkv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  // (the position by a vector load ahead of all others: a scalar one would be waited for with the arguments; without a
+  // pointer it reads the workspace and drops what it finds)
+  const int64_t pv = __hip_atomic_load(pos_ptr ? pos_ptr : (const int64_t*)part, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   const int wq = w & 3;
   const float* src = qkv + (wq < 2 ? (2 * kvh + wq) * SK_HD : nq * SK_HD + ((wq - 2) * nkv + kvh) * SK_HD);
   const float* nw = wq < 2 ? qn : kn;
