@@ -795,12 +795,14 @@ class Qwen3Kernels(Qwen3Fast):
         from . import prefill
 
         pre = prefill.plan(self.talker.model, self.T, self.kc, self.vc, L)
-        if pre is not None and prefill.agrees(pre, self._prefill_run, self.kc, self.vc):
-            def own(embeds, cpos):
-                self.tcache.seek(L)  # where the modules leave it
-                return pre(embeds)
+        if pre is not None and not prefill.agrees(pre, self._prefill_run, self.kc, self.vc):
+            pre = None
 
-            self._prefill_own = own
+        def own(embeds, cpos):
+            self.tcache.seek(L)  # where the modules leave it
+            return pre(embeds)
+
+        self._prefill_own = own if pre is not None else None
         try:
             return (*super()._capture_prefill(L)[:3], pre)
         finally:

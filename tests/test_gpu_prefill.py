@@ -114,15 +114,17 @@ def _engine(gpu, L):
     return eng, torch.from_numpy(syn.prompt_embeds(5, s, L)).to(gpu).to(torch.bfloat16)
 
 
-@pytest.mark.parametrize("other", [False, True])
-def test_recorded_prefill_is_the_modules(gpu, other):
+@pytest.mark.parametrize("other", ["", "scale", "probe"])
+def test_recorded_prefill_is_the_modules(gpu, monkeypatch, other):
     """An engine over bf16 modules records the prompt on the package's kernels, or through the modules where they name another
-    attention scale. Either way the graph's results are the modules' within two bf16 evaluations, replays repeat them,
+    attention scale or the probe disagrees. Either way the graph's results are the modules' within two bf16 evaluations, replays repeat them,
     and the transformers cache stands at the prompt's end."""
     L = 21
-    print(f"recorded prefill, another scale: {other}", flush=True)
+    print(f"recorded prefill, left to the modules by: {other or 'nothing'}", flush=True)
     eng, emb = _engine(gpu, L)
-    if other:
+    if other == "probe":
+        monkeypatch.setattr(prefill, "agrees", lambda *a: False)
+    if other == "scale":
         for y in eng.talker.model.layers:
             y.self_attn.scaling *= 1.5
     with torch.no_grad():
@@ -131,7 +133,7 @@ def test_recorded_prefill_is_the_modules(gpu, other):
     for _ in range(2):
         eng._prefill(emb)
         torch.cuda.synchronize()
-        assert (eng._pf[L][3] is None) == other
+        assert (eng._pf[L][3] is None) == bool(other)
         assert _rel(eng.ph32, ref[0, -1].double().cpu()) < 2e-2
         assert _rel(eng.kc[:, :, :L], rk[:, :, :L].double().cpu()) < 2e-2 and _rel(eng.vc[:, :, :L], rv[:, :, :L].double().cpu()) < 2e-2
         assert int(eng.pos) == L and all(int(y.cumulative_length) == L for y in eng.tcache.layers)
